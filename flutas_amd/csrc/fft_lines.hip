@@ -509,12 +509,13 @@ int LineTables::build(int n_) {
 void LineTables::release() {
   for (void *p : {(void *)d_tw, (void *)d_twh, (void *)d_twq, (void *)f_tw,
                   (void *)f_twh, (void *)f_twq, (void *)d_ptw, (void *)f_ptw,
-                  (void *)d_twe, (void *)f_twe, (void *)d_t4, (void *)f_t4})
+                  (void *)d_twe, (void *)f_twe, (void *)d_t4, (void *)f_t4,
+                  (void *)d_gen, (void *)f_gen})
     if (p) (void)hipFree(p);
   d_tw = d_twh = d_twq = d_twe = d_t4 = nullptr;
   f_tw = f_twh = f_twq = f_twe = f_t4 = nullptr;
-  d_ptw = nullptr;
-  f_ptw = nullptr;
+  d_ptw = d_gen = nullptr;
+  f_ptw = f_gen = nullptr;
 }
 
 template <typename T, typename Tin, typename Tout>

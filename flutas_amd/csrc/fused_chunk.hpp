@@ -67,6 +67,80 @@ __device__ __forceinline__ void zc_slab_of(int nx, int nchunk, int *i, int *ch) 
   }
 }
 
+// Forward elimination of one column over the np rows k0.. of a plane group:
+// y holds the rows' values and receives pL (rows past np repeat the last
+// one); dp, pp carry the pivot factor and the value, w, S, E the chunk's sums, ym the closing
+// plane of periodic z.
+// Regular rows run straight through: the coefficients and values are loaded
+// ahead, eight rows at a time (scalar registers), and no branch separates the
+// rows, so that what remains is the chain of pivots.
+template <typename T, int GP, bool PER>
+__device__ __forceinline__ void zc_eliminate(const double *__restrict__ a,
+                                             const double *__restrict__ b,
+                                             const double *__restrict__ c, int k0, int np,
+                                             int msys, int pin, double lam, T *y, double &dp,
+                                             double &pp, double &w, double &S, double &E,
+                                             double &ym) {
+#pragma clang fp contract(off)
+  if (k0 > 0 && k0 + GP < msys && np == GP) {
+    constexpr int H = GP < 8 ? GP : 8;
+#pragma unroll
+    for (int h = 0; h < GP; h += H) {
+      double av[H], bv[H], cv[H];
+#pragma unroll
+      for (int l = 0; l < H; ++l) {
+        av[l] = a[k0 + h + l];
+        bv[l] = b[k0 + h + l];
+        cv[l] = c[k0 + h + l];
+      }
+#pragma unroll
+      for (int l = 0; l < H; ++l) {
+        const double z = zrcp<T>((bv[l] + lam) - av[l] * dp);
+        dp = cv[l] * z;
+        pp = ((double)y[h + l] - av[l] * pp) * z;
+        y[h + l] = (T)pp;
+        // the sums see the stored (rounded) values P3 reads back
+        S = S + w * (double)y[h + l];
+        w = -(dp * w);
+      }
+    }
+    E = (double)y[GP - 1];
+    return;
+  }
+#pragma unroll
+  for (int l = 0; l < GP; ++l) {
+    if (l >= np) {
+      y[l] = y[l > 0 ? l - 1 : 0];
+      continue;
+    }
+    const int k = k0 + l;
+    const double ak = k == 0 ? 0.0 : a[k];
+    const double den = (b[k] + lam) - ak * dp;
+    const double num = (double)y[l] - ak * pp;
+    double pv, dk = 0.0;
+    if (k < msys - 1) {
+      const double z = zrcp<T>(den);
+      dk = c[k] * z;
+      dp = dk;
+      pv = num * z;
+    } else if (k == msys - 1) {
+      pv = (den != 0.0 && (PER || !(pin && lam == 0.0))) ? num / den : 0.0;
+    } else {
+      // a plane outside the system (periodic z: the closing plane)
+      pv = (double)y[l];
+      if (PER) ym = pv;
+    }
+    const T pt = (T)pv;
+    if (k < msys) {
+      S = S + w * (double)pt;
+      w = -(dk * w);
+      E = (double)pt;
+    }
+    pp = pv;
+    y[l] = pt;
+  }
+}
+
 // ---------------------------------------------------------------- P2 -----
 template <typename T, int NC, int GP, int NT, bool PER>
 __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, const ZChunks &zc,
@@ -159,51 +233,16 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
     if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false>(Z, Y, W.tq, sine);
     else tile::post_fwd_pp<T, NC, GP, NT, LS>(Z, Y, kind, W.th, W.tq);
 #pragma unroll
-    for (int l = 0; l < GP; ++l) {
-      if (l >= np) {
+    for (int u = 0; u < CPT; ++u) {
+      const int j = CPT * threadIdx.x + u;
+      if (CPT * NT != n && j >= n) continue;
+      T y[GP];
 #pragma unroll
-        for (int u = 0; u < CPT; ++u) hold[l][u] = hold[l - 1][u];
-        continue;
-      }
-      const int k = k0 + l;
-      const double ak = a[k], bk = b[k], cc = c[k];
+      for (int l = 0; l < GP; ++l) y[l] = Y[l * LS + j];
+      zc_eliminate<T, GP, PER>(a, b, c, k0, np, msys, pin, lam[u], y, dprev[u], pprev[u], w[u],
+                               S[u], E[u], ym[u]);
 #pragma unroll
-      for (int u = 0; u < CPT; ++u) {
-        const int j = CPT * threadIdx.x + u;
-        if (CPT * NT != n && j >= n) continue;
-        const double y = (double)Y[l * LS + j];
-        double pv, dk = 0.0;
-        if (k >= msys) {
-          // a plane outside the system (periodic z: the closing plane)
-          pv = y;
-          if (PER) ym[u] = y;
-        } else if (k == 0) {
-          const double z = zrcp<T>(bk + lam[u]);
-          dprev[u] = cc * z;
-          dk = dprev[u];
-          pv = y * z;
-        } else if (k < msys - 1) {
-          const double z = zrcp<T>((bk + lam[u]) - ak * dprev[u]);
-          dprev[u] = cc * z;
-          dk = dprev[u];
-          pv = (y - ak * pprev[u]) * z;
-        } else {
-          const double z = (bk + lam[u]) - ak * dprev[u];
-          if (z != 0.0 && (PER || !(pin && lam[u] == 0.0)))
-            pv = (y - ak * pprev[u]) / z;
-          else
-            pv = 0.0;
-        }
-        const T pt = (T)pv;
-        if (k < msys) {
-          // the sums see the stored (rounded) values P3 reads back
-          S[u] = S[u] + w[u] * (double)pt;
-          w[u] = -(dk * w[u]);
-          E[u] = (double)pt;
-        }
-        pprev[u] = pv;
-        hold[l][u] = pt;
-      }
+      for (int l = 0; l < GP; ++l) hold[l][u] = y[l];
     }
     __syncthreads();
   }
@@ -212,6 +251,181 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
   store_cols<double, CPT, NT>(sd, E, n);
   store_cols<double, CPT, NT>(sd + n, S, n);
   if (PER && ch == zc.nchunk - 1) store_cols<double, CPT, NT>(sd + 2 * n, ym, n);
+}
+
+// The reduced system of a slab's chunks, for the CPT columns of a thread (n
+// columns per line): the carry into chunk ch (Pc), x of the plane after it
+// (pn), for periodic z also p2 of that plane (pn2) and the closing plane's
+// value (xm).  Pc, pn, pn2, xm come in as zeros; get(line, v) loads the
+// thread's columns of a line.
+template <int CPT, bool PER, typename G>
+__device__ __forceinline__ void zc_carries(const ZChunks &zc, int n, int nch, int i, int ch,
+                                           int nz, const double *__restrict__ a,
+                                           const double *__restrict__ b,
+                                           const double *__restrict__ c, int pin,
+                                           const double *lam, double *Pc, double *pn,
+                                           double *pn2, double *xm, G get) {
+#pragma clang fp contract(off)
+  constexpr int TS = zc_tab_slots(PER), SS = zc_side_slots(PER);
+  const double *tb = zc.tab + (long long)i * nch * TS * n;
+  const double *sd = zc.side + (long long)i * nch * SS * n;
+  double Pk[kMaxZChunks][CPT], Pv[CPT], X[CPT];
+#pragma unroll
+  for (int u = 0; u < CPT; ++u) {
+    Pv[u] = 0.0;
+    X[u] = 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < kMaxZChunks; ++q) {
+    if (q >= nch) break;
+    double Eq[CPT], Mq[CPT];
+    get(sd + (long long)q * SS * n, Eq);
+    get(tb + (long long)q * TS * n, Mq);
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+      Pk[q][u] = Pv[u];
+      Pv[u] = Eq[u] + Mq[u] * Pv[u];
+    }
+  }
+#pragma unroll
+  for (int q = kMaxZChunks - 1; q >= 0; --q) {
+    if (q >= nch) continue;
+    double Sq[CPT], SWq[CPT], Nq[CPT];
+    get(sd + ((long long)q * SS + 1) * n, Sq);
+    get(tb + ((long long)q * TS + 1) * n, SWq);
+    get(tb + ((long long)q * TS + 2) * n, Nq);
+#pragma unroll
+    for (int u = 0; u < CPT; ++u) {
+      if (q == ch) {
+        pn[u] = X[u];
+        Pc[u] = Pk[q][u];
+      }
+      X[u] = (Sq[u] + Pk[q][u] * SWq[u]) + Nq[u] * X[u];
+    }
+  }
+  if constexpr (PER) {
+    // Pv: p1 of row m-1; X: p1(0)
+    const int m = nz - 1;
+    double Ym[CPT], Dn[CPT];
+    get(sd + ((long long)(nch - 1) * SS + 2) * n, Ym);
+    get(zc.den + (long long)i * n, Dn);
+    if (ch < nch - 1) get(tb + ((long long)ch * TS + 3) * n, pn2);
+#pragma unroll
+    for (int u = 0; u < CPT; ++u)
+      xm[u] = (pin && lam[u] == 0.0) ? 0.0 : (Ym[u] - c[m] * X[u] - a[m] * Pv[u]) / Dn[u];
+  }
+}
+
+// Back substitution of one column over the np rows k0.. of a plane group:
+// d, m (periodic: q2) of its rows recomputed from the values before it (dp,
+// mp, qp), then x(k) = pL(k) + m(k) Pc - d(k) x(k+1) downwards; pv(l) gives
+// row l's value, replaced by the solution; pn, pn2 carry to the next group.
+template <typename T, int GP, bool PER, typename F>
+__device__ __forceinline__ void zc_substitute(const double *__restrict__ a,
+                                              const double *__restrict__ b,
+                                              const double *__restrict__ c, int k0, int np,
+                                              int msys, int pin, double lam, double dp, double mp,
+                                              double qp, double Pc, double xm, double &pn,
+                                              double &pn2, F pv) {
+#pragma clang fp contract(off)
+  double d[GP], mm[GP], q2[GP];
+  double xn = pn, xn2 = pn2;
+  // A group of regular rows (not the first, none at or past the last of the
+  // system) runs straight through, see zc_eliminate.
+  if (k0 > 0 && k0 + GP < msys && np == GP) {
+    constexpr int H = GP < 8 ? GP : 8;
+#pragma unroll
+    for (int h = 0; h < GP; h += H) {
+      double av[H], bv[H], cv[H];
+#pragma unroll
+      for (int l = 0; l < H; ++l) {
+        av[l] = a[k0 + h + l];
+        bv[l] = b[k0 + h + l];
+        cv[l] = c[k0 + h + l];
+      }
+#pragma unroll
+      for (int l = 0; l < H; ++l) {
+        const double z = zrcp<T>((bv[l] + lam) - av[l] * dp);
+        dp = cv[l] * z;
+        mp = (-av[l] * mp) * z;
+        if (PER) qp = (0.0 - av[l] * qp) * z;
+        d[h + l] = dp;
+        mm[h + l] = mp;
+        q2[h + l] = qp;
+      }
+    }
+#pragma unroll
+    for (int l = GP - 1; l >= 0; --l) {
+      const double p1 = ((double)pv(l) + mm[l] * Pc) - d[l] * xn;
+      xn = p1;
+      if constexpr (PER) {
+        xn2 = q2[l] - d[l] * xn2;
+        pv(l) = (T)(p1 + xn2 * xm);
+      } else {
+        pv(l) = (T)p1;
+      }
+    }
+    pn = xn;
+    pn2 = xn2;
+    return;
+  }
+#pragma unroll
+  for (int l = 0; l < GP; ++l) {
+    const int k = k0 + l;
+    double dl = 0.0, ml = 0.0;
+    if (l < np && k < msys) {
+      const double ak = k == 0 ? 0.0 : a[k];
+      const double r2 = (k == msys - 1) ? -c[k] : ((k == 0) ? -a[0] : 0.0);
+      const double den = (b[k] + lam) - ak * dp;
+      if (k < msys - 1) {
+        const double z = zrcp<T>(den);
+        dp = c[k] * z;
+        mp = (-ak * mp) * z;
+        if (PER) qp = (r2 - ak * qp) * z;
+        dl = dp;
+      } else {
+        mp = (den != 0.0 && (PER || !(pin && lam == 0.0))) ? (-ak * mp) / den : 0.0;
+        if (PER) qp = (den != 0.0) ? (r2 - ak * qp) / den : 0.0;
+      }
+      ml = mp;
+    }
+    d[l] = dl;
+    mm[l] = ml;
+    q2[l] = qp;
+  }
+#pragma unroll
+  for (int l = GP - 1; l >= 0; --l) {
+    if (l >= np) continue;
+    const int k = k0 + l;
+    const double pt = (double)pv(l);
+    double x;
+    if constexpr (!PER) {
+      if (k >= msys) x = pt;
+      else if (k == msys - 1) x = pt + mm[l] * Pc;
+      else x = (pt + mm[l] * Pc) - d[l] * xn;
+      xn = x;
+    } else {
+      if (k >= msys) {
+        x = xm;
+      } else {
+        const double p1t = pt + mm[l] * Pc;
+        double p1, p2;
+        if (k == msys - 1) {
+          p1 = p1t;
+          p2 = q2[l];
+        } else {
+          p1 = p1t - d[l] * xn;
+          p2 = q2[l] - d[l] * xn2;
+        }
+        xn = p1;
+        xn2 = p2;
+        x = p1 + p2 * xm;
+      }
+    }
+    pv(l) = (T)x;
+  }
+  pn = xn;
+  pn2 = xn2;
 }
 
 // ---------------------------------------------------------------- P3 -----
@@ -252,64 +466,12 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
     const int j = CPT * threadIdx.x + u;
     lam[u] = (j < n) ? lx + lamy[j] : 0.0;
   }
-  // The reduced system of the slab's chunks: carry into this chunk (Pc),
-  // x of the plane after it (pn), periodic: p2 of that plane (pn2) and the
-  // closing plane's value (xm).
   double Pc[CPT], pn[CPT], pn2[CPT], xm[CPT];
-  {
-    constexpr int TS = zc_tab_slots(PER), SS = zc_side_slots(PER);
-    const double *tb = zc.tab + (long long)i * nch * TS * n;
-    const double *sd = zc.side + (long long)i * nch * SS * n;
-    double Pk[kMaxZChunks][CPT], Pv[CPT], X[CPT];
 #pragma unroll
-    for (int u = 0; u < CPT; ++u) {
-      Pv[u] = 0.0;
-      X[u] = 0.0;
-      Pc[u] = 0.0;
-      pn[u] = 0.0;
-      pn2[u] = 0.0;
-      xm[u] = 0.0;
-    }
-#pragma unroll
-    for (int q = 0; q < kMaxZChunks; ++q) {
-      if (q >= nch) break;
-      double Eq[CPT], Mq[CPT];
-      load_cols<double, CPT, NT>(sd + (long long)q * SS * n, Eq, n);
-      load_cols<double, CPT, NT>(tb + (long long)q * TS * n, Mq, n);
-#pragma unroll
-      for (int u = 0; u < CPT; ++u) {
-        Pk[q][u] = Pv[u];
-        Pv[u] = Eq[u] + Mq[u] * Pv[u];
-      }
-    }
-#pragma unroll
-    for (int q = kMaxZChunks - 1; q >= 0; --q) {
-      if (q >= nch) continue;
-      double Sq[CPT], SWq[CPT], Nq[CPT];
-      load_cols<double, CPT, NT>(sd + ((long long)q * SS + 1) * n, Sq, n);
-      load_cols<double, CPT, NT>(tb + ((long long)q * TS + 1) * n, SWq, n);
-      load_cols<double, CPT, NT>(tb + ((long long)q * TS + 2) * n, Nq, n);
-#pragma unroll
-      for (int u = 0; u < CPT; ++u) {
-        if (q == ch) {
-          pn[u] = X[u];
-          Pc[u] = Pk[q][u];
-        }
-        X[u] = (Sq[u] + Pk[q][u] * SWq[u]) + Nq[u] * X[u];
-      }
-    }
-    if constexpr (PER) {
-      // Pv: p1 of row m-1; X: p1(0)
-      const int m = nz - 1;
-      double Ym[CPT], Dn[CPT];
-      load_cols<double, CPT, NT>(sd + ((long long)(nch - 1) * SS + 2) * n, Ym, n);
-      load_cols<double, CPT, NT>(zc.den + (long long)i * n, Dn, n);
-      if (ch < nch - 1) load_cols<double, CPT, NT>(tb + ((long long)ch * TS + 3) * n, pn2, n);
-#pragma unroll
-      for (int u = 0; u < CPT; ++u)
-        xm[u] = (pin && lam[u] == 0.0) ? 0.0 : (Ym[u] - c[m] * X[u] - a[m] * Pv[u]) / Dn[u];
-    }
-  }
+  for (int u = 0; u < CPT; ++u) Pc[u] = pn[u] = pn2[u] = xm[u] = 0.0;
+  zc_carries<CPT, PER>(
+      zc, n, nch, i, ch, nz, a, b, c, pin, lam, Pc, pn, pn2, xm,
+      [](const double *line, double *v) { load_cols<double, CPT, NT>(line, v, n); });
   T pv[GP][CPT];
   double dck[CPT], mck[CPT], qck[CPT];
   auto load = [&](int g) {
@@ -350,72 +512,9 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
     for (int u = 0; u < CPT; ++u) {
       const int j = CPT * threadIdx.x + u;
       if (CPT * NT != n && j >= n) continue;
-      // d, m (periodic: q2) of the group's rows from the values before it
-      double d[GP], mm[GP], q2[GP];
-      double dp = dck[u], mp = mck[u], qp = PER ? qck[u] : 0.0;
-#pragma unroll
-      for (int l = 0; l < GP; ++l) {
-        const int k = k0 + l;
-        double dl = 0.0, ml = 0.0;
-        if (l < np && k < msys) {
-          const double r2 = PER ? ((k == msys - 1) ? -c[msys - 1] : ((k == 0) ? -a[0] : 0.0)) : 0.0;
-          if (k == 0) {
-            const double z = zrcp<T>(b[0] + lam[u]);
-            dp = c[0] * z;
-            mp = 0.0;
-            if (PER) qp = r2 * z;
-            dl = dp;
-          } else if (k < msys - 1) {
-            const double z = zrcp<T>((b[k] + lam[u]) - a[k] * dp);
-            dp = c[k] * z;
-            mp = (-a[k] * mp) * z;
-            if (PER) qp = (r2 - a[k] * qp) * z;
-            dl = dp;
-          } else {
-            const double z = (b[k] + lam[u]) - a[k] * dp;
-            mp = (z != 0.0 && (PER || !(pin && lam[u] == 0.0))) ? (-a[k] * mp) / z : 0.0;
-            if (PER) qp = (z != 0.0) ? (r2 - a[k] * qp) / z : 0.0;
-          }
-          ml = mp;
-        }
-        d[l] = dl;
-        mm[l] = ml;
-        q2[l] = qp;
-      }
-      double xn = pn[u], xn2 = pn2[u];
-#pragma unroll
-      for (int l = GP - 1; l >= 0; --l) {
-        if (l >= np) continue;
-        const int k = k0 + l;
-        const double pt = (double)pv[l][u];
-        double x;
-        if constexpr (!PER) {
-          if (k >= msys) x = pt;
-          else if (k == msys - 1) x = pt + mm[l] * Pc[u];
-          else x = (pt + mm[l] * Pc[u]) - d[l] * xn;
-          xn = x;
-        } else {
-          if (k >= msys) {
-            x = xm[u];
-          } else {
-            const double p1t = pt + mm[l] * Pc[u];
-            double p1, p2;
-            if (k == msys - 1) {
-              p1 = p1t;
-              p2 = q2[l];
-            } else {
-              p1 = p1t - d[l] * xn;
-              p2 = q2[l] - d[l] * xn2;
-            }
-            xn = p1;
-            xn2 = p2;
-            x = p1 + p2 * xm[u];
-          }
-        }
-        pv[l][u] = (T)x;
-      }
-      pn[u] = xn;
-      pn2[u] = xn2;
+      zc_substitute<T, GP, PER>(
+          a, b, c, k0, np, msys, pin, lam[u], dck[u], mck[u], PER ? qck[u] : 0.0, Pc[u], xm[u],
+          pn[u], pn2[u], [&](int l) -> T & { return pv[l][u]; });
     }
     if (g + 1 < ge) {
       flush(g + 1);

@@ -66,6 +66,19 @@ struct LinePlan {
   const T *t4;
 };
 
+// Radix list and launch shape of the general kernels (general.hip) for one
+// length: x tiles (2^lgL lines) and slab groups (gp planes, cpt columns per
+// thread).
+constexpr int kGenMaxPass = 10;
+struct RadixList {
+  int r[kGenMaxPass];
+  int nst = kGenMaxPass + 1;
+};
+struct GenShape {
+  int lgL = -1, gp = 0, cpt = 0, nt = 0;
+  RadixList rl;
+};
+
 // Host-owned device tables for one length, in double and float.
 struct LineTables {
   int n = 0, N = 0, nst = 0;
@@ -78,6 +91,11 @@ struct LineTables {
   // build_fused_twiddles when the length has a compiled plan)
   double *d_ptw = nullptr;
   float *f_ptw = nullptr;
+  // staged tables of the general kernels (set by build_general_tables for
+  // lengths without a compiled plan)
+  double *d_gen = nullptr;
+  float *f_gen = nullptr;
+  GenShape gen_x[2], gen_y;  // x tiles in FP64 and FP32, slab groups
   LinePlan<double> dplan() const;
   LinePlan<float> fplan() const;
   int build(int n);
@@ -130,8 +148,15 @@ struct WStride {
 __host__ __device__ inline WStride slab_blocked(int ny, int nz, int lb) {
   return {(long long)nz * ny << lb, ny, (long long)ny << lb, lb};
 }
-__host__ __device__ inline WStride plane_major(int nx, int ny) {
-  return {0, ny, (long long)nx * ny, 30};
+// Distance of the y-lines: whole 128-byte lines (16 FP64, 32 FP32 values)
+// for lines of 64 points and more, so that the row pieces an x tile of 16
+// lines writes do not straddle them.
+__host__ __device__ inline int line_pitch(int ny, int elem_bytes) {
+  const int q = 128 / elem_bytes;
+  return ny < 64 ? ny : (ny + q - 1) / q * q;
+}
+__host__ __device__ inline WStride plane_major(int nx, int pitch) {
+  return {0, pitch, (long long)nx * pitch, 30};
 }
 // The layout of the FP64 single solve.  Measured on one MI355X: with
 // 512-point y-lines (4 KB rows; 512^3), blocks of 4 to 128 slabs run the
@@ -141,7 +166,7 @@ __host__ __device__ inline WStride plane_major(int nx, int ny) {
 // refined mode is 2% faster plane-major, and the batched solves measure the
 // same either way (they stay plane-major).
 __host__ __device__ inline WStride fused_layout_fp64(int nx, int ny, int nz) {
-  if (ny != 512) return plane_major(nx, ny);
+  if (ny != 512) return plane_major(nx, line_pitch(ny, 8));
   int lb = 0;
   while (lb < 3 && ((nx >> lb) & 1) == 0) ++lb;
   return slab_blocked(ny, nz, lb);
@@ -211,6 +236,32 @@ int launch_zy_bwd(const LineTables &ty, int kind, T *Wt, WStride ws,
                   const double *ck, int nx, int nz, int nzs, const double *lamx,
                   const double *lamy, const double *a, const double *b,
                   const double *c, int periodic, hipStream_t s);
+
+// ---- the four passes at run-time line lengths (general.hip) --------------
+// Every even length the tile shapes reach (2..2048) that has no compiled
+// plan.  The passes take the arguments of the compiled ones; the slab passes
+// are always z-chunked (zc.nchunk >= 1), in groups of general_group_planes(ny).
+bool general_supported(int n);
+int general_group_planes(int ny);
+int general_slab_residency(int ny, int elem_bytes, int periodic, int *r2, int *r3);
+int build_general_tables(LineTables &tab, int n);
+int gen_x_fwd_blocks(int n, int elem_bytes, int ny, int nz);
+template <typename T, typename Tin>
+int launch_gen_x_fwd(const LineTables &tx, int kind, const Tin *in, long long is1, long long is2,
+                     T *Wt, WStride ws, int ny, int nz, double *absmax_part, int *nf_flag,
+                     int nf_seq, hipStream_t s);
+template <typename T, typename Tout>
+int launch_gen_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws, Tout *out,
+                     long long os1, long long os2, int ny, int nz, T scale, int accumulate,
+                     hipStream_t s);
+template <typename T>
+int launch_gen_yz_fwd(const LineTables &ty, int kind, T *Wt, WStride ws, const ZChunks &zc, int nx,
+                      int nz, int msys, const double *lamx, const double *lamy, const double *a,
+                      const double *b, const double *c, int pin, int periodic, hipStream_t s);
+template <typename T>
+int launch_gen_zy_bwd(const LineTables &ty, int kind, T *Wt, WStride ws, const ZChunks &zc, int nx,
+                      int nz, int msys, const double *lamx, const double *lamy, const double *a,
+                      const double *b, const double *c, int pin, int periodic, hipStream_t s);
 
 // ---- batched pipeline: one persistent launch over a work queue ---------
 // Stages of the batched solve (see batch.hip): the four passes of a solve,

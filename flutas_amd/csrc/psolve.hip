@@ -161,7 +161,9 @@ struct flutas_psolve {
   // [nres, nres + nx1) max|f| of the FP32 P1, then two result slots
   double *part = nullptr;
   size_t nres = 0, nx1 = 0;
-  bool fused = false;      // four-pass pipeline (fused.hip) in use
+  bool fused = false;      // four-pass pipeline (fused.hip, general.hip) in use
+  bool gx = false, gy = false;  // x / y lines on the kernels of general.hip
+  bool compiled() const { return fused && !gx && !gy; }
   double *CK = nullptr;    // z elimination checkpoints of the fused pipeline
   // z-chunked slab passes (fused_chunk.hpp): chunks per x-slab (1: whole
   // slabs), their tables, and the element size of the chain they serve
@@ -185,6 +187,11 @@ struct flutas_psolve {
 };
 
 namespace {
+
+// Values of a work field (see line_pitch).
+size_t work_values(const flutas_psolve *h, int elem_bytes) {
+  return (size_t)h->nx * line_pitch(h->ny, elem_bytes) * h->nz;
+}
 
 template <typename T>
 int dev_upload(T **d, const std::vector<T> &h) {
@@ -290,6 +297,10 @@ int zsolve(flutas_psolve *h, T *W, hipStream_t s) {
 // has chunk tables for this chain's element size, whole slabs otherwise.
 template <typename T>
 int slab_fwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s) {
+  if (h->gy)
+    return launch_gen_yz_fwd<T>(h->ty, h->kinds[2], W, ws, h->zc, h->nx, h->nz,
+                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
+                                h->d_c, pin, per, s);
   if (h->zchunks > 1 && h->zc_elem == (int)sizeof(T))
     return launch_yz_fwd_zc<T>(h->ty, h->kinds[2], W, ws, h->zc, h->nx, h->nz,
                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
@@ -299,12 +310,31 @@ int slab_fwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s
 }
 template <typename T>
 int slab_bwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s) {
+  if (h->gy)
+    return launch_gen_zy_bwd<T>(h->ty, h->kinds[3], W, ws, h->zc, h->nx, h->nz,
+                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
+                                h->d_c, pin, per, s);
   if (h->zchunks > 1 && h->zc_elem == (int)sizeof(T))
     return launch_zy_bwd_zc<T>(h->ty, h->kinds[3], W, ws, h->zc, h->nx, h->nz,
                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
                                h->d_c, pin, per, s);
   return launch_zy_bwd<T>(h->ty, h->kinds[3], W, ws, h->CK, h->nx, h->nz, h->nzs, h->d_lamx,
                           h->d_lamy, h->d_a, h->d_b, h->d_c, per, s);
+}
+
+// Planes per chunk when nz planes are cut into n chunks or fewer: a multiple
+// of the plane group gp near nz / n, rounded up where rounding to the nearest
+// would leave a longer last chunk (90 planes in 8 chunks of 8: 34 in the
+// last one; in 6 of 16: 10).
+void chunk_shape(int nz, int gp, int n, int *cpl, int *nch) {
+  *cpl = gp * std::max(1, (nz / n + gp / 2) / gp);
+  *nch = std::min(n, (nz + *cpl - 1) / *cpl);
+  const int up = gp * ((nz + n * gp - 1) / (n * gp));
+  if (std::max(*cpl, nz - (*nch - 1) * *cpl) > up) {
+    *cpl = up;
+    *nch = (nz + up - 1) / up;
+  }
+  while (*nch > 1 && (*nch - 1) * *cpl > nz - 2) --*nch;
 }
 
 // Chunks per x-slab for the z-chunked slab passes: n = 1 turns them off.
@@ -321,17 +351,15 @@ int set_zchunks(flutas_psolve *h, int n) {
   h->zchunks = 1;
   h->zc = ZChunks{};
   h->zc_elem = 0;
-  if (n == 1 || !h->fused) return FLUTAS_OK;
+  if (!h->fused || (n == 1 && !h->gy)) return FLUTAS_OK;
   const int elem = (h->precision == FLUTAS_FP64) ? 8 : 4;
-  const int gp = fused_group_planes(h->ny, elem);
+  const int gp = h->gy ? general_group_planes(h->ny) : fused_group_planes(h->ny, elem);
   const int nz = h->nz;
   const int per = (h->cbc[4] == 'P');
   const int pin = (h->cbc[4] == 'N' && h->cbc[5] == 'N') || per;
-  // planes per chunk: a multiple of gp near nz / n
-  const int cpl = gp * std::max(1, (nz / n + gp / 2) / gp);
-  int nch = std::min(n, (nz + cpl - 1) / cpl);
-  while (nch > 1 && (nch - 1) * cpl > nz - 2) --nch;
-  if (nch < 2) return FLUTAS_OK;
+  int cpl, nch;
+  chunk_shape(nz, gp, n, &cpl, &nch);
+  if (nch < 2 && !h->gy) return FLUTAS_OK;
   const int ngrp = (nz + gp - 1) / gp;
   const size_t nd = zchunk_doubles(h->nx, h->ny, ngrp, nch, per != 0);
   FL_HIP(hipMalloc((void **)&h->zc_mem, nd * sizeof(double)));
@@ -355,7 +383,14 @@ int set_zchunks(flutas_psolve *h, int n) {
 // the GPU holds at once (CUs x residency per CU from the occupancy
 // calculator), runs ceil(W / R) rounds and keeps W / (ceil(W / R) R) of
 // the slots busy; the score is the mean of that fill over P2 and P3, ties
-// go to the smaller count, and every chunk keeps 32 planes or more.  The
+// go to the smaller count.  A chunk keeps 32 planes or more (two plane groups
+// on the general kernels), or one plane group where the workgroups do not
+// reach the number of CUs: a pass of so few is the walk of one workgroup
+// (64^3: 2 chunks 31.3 us, 4 of one group 25.6; 2x64x64: 30.2, 25.1; 72x60x50
+// 58.6 for 3, 50.6 for 4; but 128^3 in 8 chunks of one group, 1024 workgroups,
+// 71.6 against 58.2 for 4).  The general kernels pay 0.02 per chunk
+// (528x528x128: 1.32, 1.27, 1.29, 1.38, 1.37 ms for 2, 3, 4, 6, 8; the
+// unpenalised score took 8).  The
 // FP32 chain of the refined mode pays 0.05 of score per chunk beyond the
 // first: its chunk tables and side arrays stay FP64 against half the field
 // bytes, so a chunk costs it relatively more (refined 256x256x512
@@ -377,7 +412,9 @@ int default_zchunks(const flutas_psolve *h) {
   const int elem = (h->precision == FLUTAS_FP64) ? 8 : 4;
   const int per = (h->cbc[4] == 'P');
   int r2 = 0, r3 = 0, dev = 0, ncu = 0;
-  if (fused_slab_residency(h->ny, elem, per, &r2, &r3) != FLUTAS_OK || r2 < 1 || r3 < 1 ||
+  const int rc = h->gy ? general_slab_residency(h->ny, elem, per, &r2, &r3)
+                       : fused_slab_residency(h->ny, elem, per, &r2, &r3);
+  if (rc != FLUTAS_OK || r2 < 1 || r3 < 1 ||
       hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
       ncu < 1) {
@@ -390,11 +427,16 @@ int default_zchunks(const flutas_psolve *h) {
   };
   int best = 1;
   double best_score = -1.0;
+  const int gp = h->gy ? general_group_planes(h->ny) : fused_group_planes(h->ny, elem);
   for (int n = 1; n <= kMaxZChunks; ++n) {
-    if (n > 1 && h->nz / n < 32) break;
+    int cpl, nch;
+    chunk_shape(h->nz, gp, n, &cpl, &nch);
+    if (nch != n) continue;
     const long long w = (long long)h->nx * n;
+    const int least = w <= ncu ? gp : (h->gy ? 2 * gp : 32);
+    if (n > 1 && cpl < least) break;
     const double score = 0.5 * (fill(w, (long long)ncu * r2) + fill(w, (long long)ncu * r3)) -
-                         (elem == 4 ? 0.05 * (n - 1) : 0.0);
+                         (elem == 4 ? 0.05 : (h->gy ? 0.02 : 0.0)) * (n - 1);
     if (score > best_score + 1e-9) {
       best_score = score;
       best = n;
@@ -420,16 +462,25 @@ int spectral(flutas_psolve *h, const Tin *in, bool in_halo, Tout *out,
     // the singular column takes p(last) = 0 for NN and for periodic z
     const int per = (h->cbc[4] == 'P');
     const int pin = (h->cbc[4] == 'N' && h->cbc[5] == 'N') || per;
-    const WStride ws = sizeof(T) == 8 ? fused_layout_fp64(nx, ny, nz) : plane_major(nx, ny);
-    FL_TRY((launch_x_fwd<T, Tin>(h->tx, h->kinds[0], in, is1, is2, W, ws, ny, nz, absmax_part,
-                                 nf_flag, h->seq, s)));
+    const WStride ws = sizeof(T) == 8 ? fused_layout_fp64(nx, ny, nz)
+                                      : plane_major(nx, line_pitch(ny, 4));
+    if (h->gx)
+      FL_TRY((launch_gen_x_fwd<T, Tin>(h->tx, h->kinds[0], in, is1, is2, W, ws, ny, nz,
+                                       absmax_part, nf_flag, h->seq, s)));
+    else
+      FL_TRY((launch_x_fwd<T, Tin>(h->tx, h->kinds[0], in, is1, is2, W, ws, ny, nz, absmax_part,
+                                   nf_flag, h->seq, s)));
     FL_TRY(mark(h, "P1_x_fwd", s));
     FL_TRY(slab_fwd<T>(h, W, ws, pin, per, s));
     FL_TRY(mark(h, "P2_yz_fwd", s));
     FL_TRY(slab_bwd<T>(h, W, ws, pin, per, s));
     FL_TRY(mark(h, "P3_zy_bwd", s));
-    FL_TRY((launch_x_bwd<T, Tout>(h->tx, h->kinds[1], W, ws, out, q.hx, q.hxy, ny, nz,
-                                  (T)h->normfft, accumulate, s)));
+    if (h->gx)
+      FL_TRY((launch_gen_x_bwd<T, Tout>(h->tx, h->kinds[1], W, ws, out, q.hx, q.hxy, ny, nz,
+                                        (T)h->normfft, accumulate, s)));
+    else
+      FL_TRY((launch_x_bwd<T, Tout>(h->tx, h->kinds[1], W, ws, out, q.hx, q.hxy, ny, nz,
+                                    (T)h->normfft, accumulate, s)));
     FL_TRY(mark(h, "P4_x_bwd", s));
     return FLUTAS_OK;
   }
@@ -478,13 +529,12 @@ int solve_fp64(flutas_psolve *h, const double *f, double *p, hipStream_t s) {
 // plan is an FP64 one.
 int solve_f32(flutas_psolve *h, const float *f, float *p, hipStream_t s) {
   if (!h->W32) {
-    const size_t N = (size_t)h->nx * h->ny * h->nz;
-    FL_HIP(hipMalloc((void **)&h->W32, N * sizeof(float)));
+    FL_HIP(hipMalloc((void **)&h->W32, work_values(h, 4) * sizeof(float)));
   }
   const Geo q = halo_geo(h);
   ++h->seq;
   FL_TRY((spectral<float, float, float>(h, f + q.interior, true, p + q.interior, 0, h->W32, s,
-                                        nullptr, h->fused ? h->nf_dev : nullptr)));
+                                        nullptr, h->compiled() ? h->nf_dev : nullptr)));
   h->last_iters = 0;
   h->last_relres = -1.0;
   return FLUTAS_OK;
@@ -707,10 +757,22 @@ int flutas_psolve_create(const int ng[3], const char cbc[6], const double bc[6],
   const size_t N = (size_t)h->nx * h->ny * h->nz;
   const size_t nhalo = (size_t)(h->nx + 2) * (h->ny + 2) * (h->nz + 2);
   do {
-    if ((rc = h->tx.build(h->nx))) break;
-    if ((rc = h->ty.build(h->ny))) break;
-    if (fused_supported(h->nx) && (rc = build_fused_twiddles(h->tx))) break;
-    if (fused_supported(h->ny) && (rc = build_fused_twiddles(h->ty))) break;
+    // the fused pipeline covers the compiled line lengths, and the general
+    // kernels every other even length up to 2048
+    // (the tile transforms cover the R2HC, DCT-II/III, DCT-IV and DST kinds
+    // run forward in P1/P2 and backward in P3/P4)
+    const char *env = std::getenv("FLUTAS_UNFUSED");
+    const bool tile_kinds = fused_forward_kind(h->kinds[0]) && fused_forward_kind(h->kinds[2]);
+    const bool gx = !fused_supported(h->nx), gy = !fused_supported(h->ny);
+    h->fused = (!gx || general_supported(h->nx)) && (!gy || general_supported(h->ny)) &&
+               h->nz >= 3 && tile_kinds && !(env && env[0] == '1');
+    h->gx = h->fused && gx;
+    h->gy = h->fused && gy;
+    // (a direction on the general kernels needs their tables only)
+    if ((rc = h->gx ? build_general_tables(h->tx, h->nx) : h->tx.build(h->nx))) break;
+    if ((rc = h->gy ? build_general_tables(h->ty, h->ny) : h->ty.build(h->ny))) break;
+    if (!gx && (rc = build_fused_twiddles(h->tx))) break;
+    if (!gy && (rc = build_fused_twiddles(h->ty))) break;
     if ((rc = dev_upload(&h->d_lamx, h->lamx))) break;
     if ((rc = dev_upload(&h->d_lamy, h->lamy))) break;
     if ((rc = dev_upload(&h->d_a, h->a))) break;
@@ -721,26 +783,19 @@ int flutas_psolve_create(const int ng[3], const char cbc[6], const double bc[6],
     if ((rc = dev_upload(&h->d_rhsbz, h->rhsbz))) break;
     hipError_t e = hipSuccess;
     if (precision == FLUTAS_FP64) {
-      e = hipMalloc((void **)&h->W64, N * sizeof(double));
+      e = hipMalloc((void **)&h->W64, work_values(h, 8) * sizeof(double));
     } else {
-      e = hipMalloc((void **)&h->W32, N * sizeof(float));
+      e = hipMalloc((void **)&h->W32, work_values(h, 4) * sizeof(float));
       if (e == hipSuccess) e = hipMalloc((void **)&h->R32, N * sizeof(float));
       if (e == hipSuccess) e = hipMalloc((void **)&h->F, nhalo * sizeof(double));
     }
-    // the fused pipeline covers the compiled line lengths
-    const char *env = std::getenv("FLUTAS_UNFUSED");
-    // (the tile transforms cover the R2HC, DCT-II/III and DST-II/III kinds
-    // run forward in P1/P2 and backward in P3/P4)
-    const bool tile_kinds = fused_forward_kind(h->kinds[0]) && fused_forward_kind(h->kinds[2]);
-    h->fused = fused_supported(h->nx) && fused_supported(h->ny) && h->nz >= 3 && tile_kinds &&
-               !(env && env[0] == '1');
-    if (h->fused) {
+    if (h->fused && !h->gy) {
       const int gp = fused_group_planes(h->ny, precision == FLUTAS_FP64 ? 8 : 4);
       // one checkpoint per plane group (two values per column for periodic z)
       const size_t ngrp = (h->nz + gp - 1) / gp;
       const size_t nck = std::max<size_t>(1, ngrp) * (cbc[4] == 'P' ? 2 : 1);
       if (e == hipSuccess) e = hipMalloc((void **)&h->CK, (size_t)h->nx * nck * h->ny * sizeof(double));
-    } else {
+    } else if (!h->fused) {
       const size_t ntk = thomas_checkpoint_doubles(h->nx, h->ny, h->nz, cbc[4] == 'P');
       if (e == hipSuccess) e = hipMalloc((void **)&h->TK, ntk * sizeof(double));
     }
@@ -750,7 +805,9 @@ int flutas_psolve_create(const int ng[3], const char cbc[6], const double bc[6],
       e = hipHostGetDevicePointer((void **)&h->nf_dev, h->nf_host, 0);
     }
     h->nres = residual_blocks(h->nx, h->ny, h->nz);
-    h->nx1 = (h->fused && precision == FLUTAS_FP32_REFINE) ? (size_t)x_fwd_blocks(h->tx, 4, h->ny, h->nz) : 0;
+    h->nx1 = (h->fused && precision == FLUTAS_FP32_REFINE) ? (size_t)(h->gx ? gen_x_fwd_blocks(h->nx, 4, h->ny, h->nz)
+                                           : x_fwd_blocks(h->tx, 4, h->ny, h->nz))
+                          : 0;
     if (e == hipSuccess) e = hipMalloc((void **)&h->part, (h->nres + h->nx1 + 2) * sizeof(double));
     if (e != hipSuccess) { rc = fail(FLUTAS_ENOMEM, std::string("device allocation: ") + hipGetErrorString(e)); break; }
     const char *zenv = std::getenv("FLUTAS_ZCHUNKS");
@@ -828,7 +885,7 @@ int flutas_psolve_solve_f32(flutas_psolve *h, float *p) {
   hipStream_t s = current_stream();
   FL_TRY(solve_f32(h, p, p, s));
   FL_HIP(hipStreamSynchronize(s));
-  if (h->fused && *(volatile int *)h->nf_host == h->seq)
+  if (h->compiled() && *(volatile int *)h->nf_host == h->seq)
     return fail(FLUTAS_ENONFINITE, "right-hand side holds NaN or Inf");
   return FLUTAS_OK;
 }
@@ -970,7 +1027,7 @@ int flutas_psolve_time_stage(flutas_psolve *h, const double *f, double *p, int s
                              int reps, double *ms) {
   if (!h || !f || !p || !ms || reps < 1 || reps > 16 || stage < 0 || stage > 3)
     return fail(FLUTAS_EINVAL, "bad stage timing arguments");
-  if (!h->fused || h->precision != FLUTAS_FP64)
+  if (!h->compiled() || h->precision != FLUTAS_FP64)
     return fail(FLUTAS_EUNSUPPORTED, "stage timing covers the four-pass FP64 pipeline");
   hipStream_t s = current_stream();
   FL_TRY(solve_impl(h, f, p));
