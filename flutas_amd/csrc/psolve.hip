@@ -388,10 +388,10 @@ int set_zchunks(flutas_psolve *h, int n) {
 // reach the number of CUs: a pass of so few is the walk of one workgroup
 // (64^3: 2 chunks 31.3 us, 4 of one group 25.6; 2x64x64: 30.2, 25.1; 72x60x50
 // 58.6 for 3, 50.6 for 4; but 128^3 in 8 chunks of one group, 1024 workgroups,
-// 71.6 against 58.2 for 4).  The general kernels pay 0.02 per chunk
+// 71.6 against 58.2 for 4).  The general kernels pay 2% per chunk beyond the first
 // (528x528x128: 1.32, 1.27, 1.29, 1.38, 1.37 ms for 2, 3, 4, 6, 8; the
 // unpenalised score took 8).  The
-// FP32 chain of the refined mode pays 0.05 of score per chunk beyond the
+// FP32 chain of the refined mode pays 5% of score per chunk beyond the
 // first: its chunk tables and side arrays stay FP64 against half the field
 // bytes, so a chunk costs it relatively more (refined 256x256x512
 // periodic: 1/2/3/4/6/8 chunks 1.71, 1.30, 1.36, 1.31, 1.37, 1.34 ms; the
@@ -435,8 +435,8 @@ int default_zchunks(const flutas_psolve *h) {
     const long long w = (long long)h->nx * n;
     const int least = w <= ncu ? gp : (h->gy ? 2 * gp : 32);
     if (n > 1 && cpl < least) break;
-    const double score = 0.5 * (fill(w, (long long)ncu * r2) + fill(w, (long long)ncu * r3)) -
-                         (elem == 4 ? 0.05 : (h->gy ? 0.02 : 0.0)) * (n - 1);
+    const double score = 0.5 * (fill(w, (long long)ncu * r2) + fill(w, (long long)ncu * r3)) *
+                         (1.0 - (elem == 4 ? 0.05 : (h->gy ? 0.02 : 0.0)) * (n - 1));
     if (score > best_score + 1e-9) {
       best_score = score;
       best = n;
