@@ -134,6 +134,14 @@ static bool fused_forward_kind(int k) {
 
 using namespace flutas;
 
+// One chain's z-chunked slab passes: chunks per x-slab (1: whole slabs) and
+// the tables.
+struct ChunkSet {
+  int n = 1;
+  ZChunks zc{};
+  double *mem = nullptr;
+};
+
 struct flutas_psolve {
   int nx, ny, nz;
   // planes of the z system: nz, or nz - 1 for a face-centred z grid with a
@@ -165,12 +173,12 @@ struct flutas_psolve {
   bool gx = false, gy = false;  // x / y lines on the kernels of general.hip
   bool compiled() const { return fused && !gx && !gy; }
   double *CK = nullptr;    // z elimination checkpoints of the fused pipeline
-  // z-chunked slab passes (fused_chunk.hpp): chunks per x-slab (1: whole
-  // slabs), their tables, and the element size of the chain they serve
-  int zchunks = 1;
-  ZChunks zc{};
-  double *zc_mem = nullptr;
-  int zc_elem = 0;
+  // z-chunked slab passes (fused_chunk.hpp) of the plan's own chain, and on
+  // an FP64 plan those of the FP32 solve (solve_f32), made by its first call;
+  // zreq: the chunk count asked for (0: default_zchunks)
+  ChunkSet zcs, zcs32;
+  bool has32 = false;
+  int zreq = 0;
   int last_iters = 0;
   double last_relres = -1.0;
   // NaN/Inf detection of the FP64 solve: P1 (or a flag pass on the line
@@ -206,7 +214,8 @@ void release(flutas_psolve *h) {
                   (void *)h->d_b, (void *)h->d_c, (void *)h->d_rhsbx,
                   (void *)h->d_rhsby, (void *)h->d_rhsbz, (void *)h->W64,
                   (void *)h->W32, (void *)h->TK, (void *)h->F,
-                  (void *)h->R32, (void *)h->part, (void *)h->CK, (void *)h->zc_mem})
+                  (void *)h->R32, (void *)h->part, (void *)h->CK, (void *)h->zcs.mem,
+                  (void *)h->zcs32.mem})
     if (p) (void)hipFree(p);
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   h->ev.clear();
@@ -296,13 +305,19 @@ int zsolve(flutas_psolve *h, T *W, hipStream_t s) {
 // The slab passes P2/P3 of the fused pipeline: z-chunked when the plan
 // has chunk tables for this chain's element size, whole slabs otherwise.
 template <typename T>
+const ChunkSet &chunks_of(const flutas_psolve *h) {
+  // the general kernels serve both chains from one set of tables
+  return !h->gy && sizeof(T) == 4 && h->precision == FLUTAS_FP64 ? h->zcs32 : h->zcs;
+}
+template <typename T>
 int slab_fwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s) {
+  const ChunkSet &z = chunks_of<T>(h);
   if (h->gy)
-    return launch_gen_yz_fwd<T>(h->ty, h->kinds[2], W, ws, h->zc, h->nx, h->nz,
+    return launch_gen_yz_fwd<T>(h->ty, h->kinds[2], W, ws, z.zc, h->nx, h->nz,
                                 per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
                                 h->d_c, pin, per, s);
-  if (h->zchunks > 1 && h->zc_elem == (int)sizeof(T))
-    return launch_yz_fwd_zc<T>(h->ty, h->kinds[2], W, ws, h->zc, h->nx, h->nz,
+  if (z.n > 1)
+    return launch_yz_fwd_zc<T>(h->ty, h->kinds[2], W, ws, z.zc, h->nx, h->nz,
                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
                                h->d_c, pin, per, s);
   return launch_yz_fwd<T>(h->ty, h->kinds[2], W, ws, h->CK, h->nx, h->nz, h->nzs, h->d_lamx,
@@ -310,12 +325,13 @@ int slab_fwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s
 }
 template <typename T>
 int slab_bwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s) {
+  const ChunkSet &z = chunks_of<T>(h);
   if (h->gy)
-    return launch_gen_zy_bwd<T>(h->ty, h->kinds[3], W, ws, h->zc, h->nx, h->nz,
+    return launch_gen_zy_bwd<T>(h->ty, h->kinds[3], W, ws, z.zc, h->nx, h->nz,
                                 per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
                                 h->d_c, pin, per, s);
-  if (h->zchunks > 1 && h->zc_elem == (int)sizeof(T))
-    return launch_zy_bwd_zc<T>(h->ty, h->kinds[3], W, ws, h->zc, h->nx, h->nz,
+  if (z.n > 1)
+    return launch_zy_bwd_zc<T>(h->ty, h->kinds[3], W, ws, z.zc, h->nx, h->nz,
                                per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
                                h->d_c, pin, per, s);
   return launch_zy_bwd<T>(h->ty, h->kinds[3], W, ws, h->CK, h->nx, h->nz, h->nzs, h->d_lamx,
@@ -337,22 +353,13 @@ void chunk_shape(int nz, int gp, int n, int *cpl, int *nch) {
   while (*nch > 1 && (*nch - 1) * *cpl > nz - 2) --*nch;
 }
 
-// Chunks per x-slab for the z-chunked slab passes: n = 1 turns them off.
-// The planes are cut at multiples of the plane group into n chunks (fewer
-// when nz is short; the last chunk runs to nz and holds two planes or
-// more), and the tables are computed for the plan's chain.
-int set_zchunks(flutas_psolve *h, int n) {
-  if (n < 1 || n > kMaxZChunks) return fail(FLUTAS_EINVAL, "z chunks must be 1..8");
-  if (h->zc_mem) {
-    FL_HIP(hipDeviceSynchronize());
-    (void)hipFree(h->zc_mem);
-    h->zc_mem = nullptr;
-  }
-  h->zchunks = 1;
-  h->zc = ZChunks{};
-  h->zc_elem = 0;
+// Chunks per x-slab for the z-chunked slab passes of a chain of elem-byte
+// values: n = 1 turns them off.  The planes are cut at multiples of the plane
+// group into n chunks (fewer when nz is short; the last chunk runs to nz and
+// holds two planes or more), and the tables are computed for that chain.
+int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
+  z = ChunkSet{};
   if (!h->fused || (n == 1 && !h->gy)) return FLUTAS_OK;
-  const int elem = (h->precision == FLUTAS_FP64) ? 8 : 4;
   const int gp = h->gy ? general_group_planes(h->ny) : fused_group_planes(h->ny, elem);
   const int nz = h->nz;
   const int per = (h->cbc[4] == 'P');
@@ -362,19 +369,18 @@ int set_zchunks(flutas_psolve *h, int n) {
   if (nch < 2 && !h->gy) return FLUTAS_OK;
   const int ngrp = (nz + gp - 1) / gp;
   const size_t nd = zchunk_doubles(h->nx, h->ny, ngrp, nch, per != 0);
-  FL_HIP(hipMalloc((void **)&h->zc_mem, nd * sizeof(double)));
-  const int rc = build_zchunk_tables(h->zc_mem, &h->zc, h->nx, h->ny, nz, per ? nz - 1 : h->nzs,
-                                     gp, cpl, nch, per != 0, pin, elem, h->d_lamx, h->d_lamy,
-                                     h->d_a, h->d_b, h->d_c, nullptr);
+  FL_HIP(hipMalloc((void **)&z.mem, nd * sizeof(double)));
+  const int rc = build_zchunk_tables(z.mem, &z.zc, h->nx, h->ny, nz, per ? nz - 1 : h->nzs, gp,
+                                     cpl, nch, per != 0, pin, elem, h->d_lamx, h->d_lamy, h->d_a,
+                                     h->d_b, h->d_c, nullptr);
   if (rc == FLUTAS_OK && hipDeviceSynchronize() != hipSuccess)
     return fail(FLUTAS_EDEVICE, "z chunk tables");
   if (rc) {
-    (void)hipFree(h->zc_mem);
-    h->zc_mem = nullptr;
+    (void)hipFree(z.mem);
+    z = ChunkSet{};
     return rc;
   }
-  h->zchunks = nch;
-  h->zc_elem = elem;
+  z.n = nch;
   return FLUTAS_OK;
 }
 
@@ -407,9 +413,8 @@ int set_zchunks(flutas_psolve *h, int n) {
 //   256x256x512 periodic  0.78  0.55* 0.63  0.61  0.62  0.60
 //   400^3 NN-z            1.26  1.23  1.15  1.19  1.16  1.21  (5 taken)
 // and at 128^3: 0.115, 0.082 (2), 0.065 (4, taken), 0.072 (8).
-int default_zchunks(const flutas_psolve *h) {
+int default_zchunks(const flutas_psolve *h, int elem) {
   if (!h->fused) return 1;
-  const int elem = (h->precision == FLUTAS_FP64) ? 8 : 4;
   const int per = (h->cbc[4] == 'P');
   int r2 = 0, r3 = 0, dev = 0, ncu = 0;
   const int rc = h->gy ? general_slab_residency(h->ny, elem, per, &r2, &r3)
@@ -443,6 +448,35 @@ int default_zchunks(const flutas_psolve *h) {
     }
   }
   return best;
+}
+
+// The tables of solve_f32 on an FP64 plan: its slab passes fill the GPU no
+// better than the FP64 ones (solve_f32 on whole slabs and in the default chunks:
+// 128^3 109 and 58 us, 256^3 269 and 175, 256x256x512 periodic 578 and 346,
+// 48x64x364 195 and 51; 512^3 stays at one chunk).  Whole slabs serve it
+// where the memory for them is short.
+void build_chunks32(flutas_psolve *h) {
+  if (build_chunks(h, h->zcs32, 4, h->zreq ? h->zreq : default_zchunks(h, 4)) != FLUTAS_OK) {
+    (void)hipGetLastError();
+    h->zcs32 = ChunkSet{};
+  }
+}
+
+int plan_elem(const flutas_psolve *h) { return h->precision == FLUTAS_FP64 ? 8 : 4; }
+
+// The chunk count of the plan: n for its own chain; the tables of solve_f32
+// follow zreq where they were made.
+int set_zchunks(flutas_psolve *h, int n) {
+  if (n < 1 || n > kMaxZChunks) return fail(FLUTAS_EINVAL, "z chunks must be 1..8");
+  if (h->zcs.mem || h->zcs32.mem) {
+    FL_HIP(hipDeviceSynchronize());
+    (void)hipFree(h->zcs.mem);
+    (void)hipFree(h->zcs32.mem);
+    h->zcs = h->zcs32 = ChunkSet{};
+  }
+  FL_TRY(build_chunks(h, h->zcs, plan_elem(h), n));
+  if (h->has32) build_chunks32(h);
+  return FLUTAS_OK;
 }
 
 // One spectral solve in storage/arithmetic T: the right-hand side `in`
@@ -525,11 +559,15 @@ int solve_fp64(flutas_psolve *h, const double *f, double *p, hipStream_t s) {
 // FP32: src/types.f90:6-12), in place or out of place: the FP32 chain of
 // the refined mode (FP32 transforms, FP64 z elimination) once, no
 // refinement, as the reference's single-precision solver runs its whole
-// solve in FP32.  The FP32 work field is allocated on first use when the
-// plan is an FP64 one.
+// solve in FP32.  The FP32 work field and the chunk tables are made on
+// first use when the plan is an FP64 one.
 int solve_f32(flutas_psolve *h, const float *f, float *p, hipStream_t s) {
   if (!h->W32) {
     FL_HIP(hipMalloc((void **)&h->W32, work_values(h, 4) * sizeof(float)));
+  }
+  if (!h->has32 && h->fused && !h->gy && h->precision == FLUTAS_FP64) {
+    h->has32 = true;
+    build_chunks32(h);
   }
   const Geo q = halo_geo(h);
   ++h->seq;
@@ -811,7 +849,8 @@ int flutas_psolve_create(const int ng[3], const char cbc[6], const double bc[6],
     if (e == hipSuccess) e = hipMalloc((void **)&h->part, (h->nres + h->nx1 + 2) * sizeof(double));
     if (e != hipSuccess) { rc = fail(FLUTAS_ENOMEM, std::string("device allocation: ") + hipGetErrorString(e)); break; }
     const char *zenv = std::getenv("FLUTAS_ZCHUNKS");
-    if ((rc = set_zchunks(h, zenv ? std::atoi(zenv) : default_zchunks(h)))) break;
+    h->zreq = zenv ? std::atoi(zenv) : 0;
+    if ((rc = set_zchunks(h, zenv ? h->zreq : default_zchunks(h, plan_elem(h))))) break;
   } while (0);
   if (rc) {
     release(h);
@@ -1141,12 +1180,14 @@ int flutas_event_destroy(void *ev) {
 
 int flutas_psolve_set_zchunks(flutas_psolve *h, int n) {
   if (!h) return fail(FLUTAS_EINVAL, "null plan");
-  return set_zchunks(h, n == 0 ? default_zchunks(h) : n);
+  if (n < 0 || n > kMaxZChunks) return fail(FLUTAS_EINVAL, "z chunks must be 1..8");
+  h->zreq = n;
+  return set_zchunks(h, n == 0 ? default_zchunks(h, plan_elem(h)) : n);
 }
 
 int flutas_psolve_zchunks(const flutas_psolve *h, int *n) {
   if (!h || !n) return fail(FLUTAS_EINVAL, "null pointer");
-  *n = h->zchunks;
+  *n = h->zcs.n;
   return FLUTAS_OK;
 }
 
@@ -1163,7 +1204,7 @@ int flutas_psolve_tune(flutas_psolve *h, const double *f, double *p, int reps, i
     const int n = v + 1;
     if (ms) ms[v] = -1.0;
     FL_TRY(set_zchunks(h, n));
-    if (h->zchunks != n) continue;
+    if (h->zcs.n != n) continue;
     FL_TRY(solve_impl(h, f, p));  // warm-up
     FL_HIP(hipStreamSynchronize(s));
     const auto t0 = std::chrono::steady_clock::now();
@@ -1180,7 +1221,7 @@ int flutas_psolve_tune(flutas_psolve *h, const double *f, double *p, int reps, i
   FL_TRY(set_zchunks(h, best));
   FL_TRY(solve_impl(h, f, p));
   FL_HIP(hipStreamSynchronize(s));
-  *chosen = h->zchunks;
+  *chosen = h->zcs.n;
   return check_nonfinite(h);
 }
 
