@@ -161,7 +161,7 @@ template <typename T, int NC, int GP, bool PER, int NT>
 __device__ __forceinline__ void item_yz(const BatchProblem &qin, int i) {
   const BatchProblem &q = *as_global(&qin);
   T *const dyn = lds_base<T>();
-  yz_fwd_slab<T, NC, GP, NT, PER>(as_global(static_cast<T *>(q.W)), plane_major(q.nx, q.ny),
+  yz_fwd_slab<T, NC, GP, NT, PER, false>(as_global(static_cast<T *>(q.W)), plane_major(q.nx, q.ny),
                                     as_global(q.ck), q.nx, q.nz, q.nz, q.ky_f, as_global(q.lamx),
                                     as_global(q.lamy), as_global(q.a), as_global(q.b),
                                     as_global(q.c), q.pin,
@@ -172,7 +172,7 @@ template <typename T, int NC, int GP, bool PER, int NT>
 __device__ __forceinline__ void item_zy(const BatchProblem &qin, int i) {
   const BatchProblem &q = *as_global(&qin);
   T *const dyn = lds_base<T>();
-  zy_bwd_slab<T, NC, GP, NT, PER>(as_global(static_cast<T *>(q.W)), plane_major(q.nx, q.ny),
+  zy_bwd_slab<T, NC, GP, NT, PER, false>(as_global(static_cast<T *>(q.W)), plane_major(q.nx, q.ny),
                                     as_global(q.ck), q.nx, q.nz, q.nz, q.ky_b, as_global(q.lamx),
                                     as_global(q.lamy), as_global(q.a), as_global(q.b),
                                     as_global(q.c),

@@ -373,8 +373,8 @@ struct Pair<float> {
 // pairs when CPT is even (one wide access per pair), else one by one.
 // Loads of columns past n re-read column n-1 (branch free).
 template <typename T, int CPT, int NT>
-__device__ __forceinline__ void store_cols(T *__restrict__ line, const T *v, int n) {
-  const int j0 = CPT * threadIdx.x;
+__device__ __forceinline__ void store_cols(T *__restrict__ line, const T *v, int n, int tid) {
+  const int j0 = CPT * tid;
   if constexpr (CPT % 2 == 0) {
 #pragma unroll
     for (int u = 0; u < CPT; u += 2)
@@ -391,8 +391,8 @@ __device__ __forceinline__ void store_cols(T *__restrict__ line, const T *v, int
   }
 }
 template <typename T, int CPT, int NT>
-__device__ __forceinline__ void store_cols_nt(T *__restrict__ line, const T *v, int n) {
-  const int j0 = CPT * threadIdx.x;
+__device__ __forceinline__ void store_cols_nt(T *__restrict__ line, const T *v, int n, int tid) {
+  const int j0 = CPT * tid;
   if constexpr (CPT % 2 == 0) {
 #pragma unroll
     for (int u = 0; u < CPT; u += 2)
@@ -404,8 +404,8 @@ __device__ __forceinline__ void store_cols_nt(T *__restrict__ line, const T *v, 
   }
 }
 template <typename T, int CPT, int NT>
-__device__ __forceinline__ void load_cols(const T *__restrict__ line, T *v, int n) {
-  const int j0 = CPT * threadIdx.x;
+__device__ __forceinline__ void load_cols(const T *__restrict__ line, T *v, int n, int tid) {
+  const int j0 = CPT * tid;
   if constexpr (CPT % 2 == 0) {
 #pragma unroll
     for (int u = 0; u < CPT; u += 2) {
@@ -454,7 +454,7 @@ __host__ __device__ constexpr int checkpoints(int nz) {
 
 // The slab body (also used by the batched kernels): sm holds 2*GP lines
 // of line_stride<T, ny>() elements, stw the staged twiddles.
-template <typename T, int NC, int GP, int NT, bool PER>
+template <typename T, int NC, int GP, int NT, bool PER, bool OPQ>
 __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
                                             double *__restrict__ ck,
                                             int nx, int nz, int nzs, int kind,
@@ -506,10 +506,10 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
   // branch-free prefetch of element pairs (16-byte loads in FP64): planes
   // past nz (last group) re-read plane nz-1
   auto load = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int t = min((int)threadIdx.x + q * NT, GP * n / 2 - 1);
+      const int t = min(tid + q * NT, GP * n / 2 - 1);
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       r[q] = *reinterpret_cast<const V2 *>(line0 + (long long)min(k0 + l, nz - 1) * pstride + e);
     }
@@ -523,26 +523,27 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
   // repeats plane np-1 and goes to the same address again.
   T hold[GP][CPT];
   auto flush = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int l = 0; l < GP; ++l)
-      store_cols_nt<T, CPT, NT>(line0 + (long long)min(k0 + l, nz - 1) * pstride, hold[l], n);
+      store_cols_nt<T, CPT, NT>(line0 + (long long)min(k0 + l, nz - 1) * pstride, hold[l], n, tid);
     // checkpoint of group g: ck[(i*nck + g)*ny + j] (periodic z: the
     // second right-hand side's p' follows at offset nx*nck*ny)
     double *cg = ck + ((long long)i * nck + g) * n;
-    store_cols<double, CPT, NT>(cg, dprev, n);
-    if constexpr (PER) store_cols<double, CPT, NT>(cg + (long long)nx * nck * n, q2prev, n);
+    store_cols<double, CPT, NT>(cg, dprev, n, tid);
+    if constexpr (PER) store_cols<double, CPT, NT>(cg + (long long)nx * nck * n, q2prev, n, tid);
   };
   load(0);
   for (int g = 0; g < ngrp; ++g) {
     const int k0 = g * GP;
     const int np = min(GP, nz - k0);
+    const int tid = tile::lane_id<OPQ>();
     // branch-free staging: Makhoul's reordering for the cosine/sine kinds
     // (e even -> e/2, e+1 -> n-1-e/2, odd entries negated for the sine
     // kinds), natural order otherwise
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int t = threadIdx.x + q * NT;
+      const int t = tid + q * NT;
       if ((GP * n / 2) % NT != 0 && t >= GP * n / 2) continue;
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       const int p0 = trig ? (e >> 1) : e;
@@ -559,10 +560,10 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
       tile::d4_pre<T, NC, GP, NT, LS, false>(A, W.th);
       __syncthreads();
     }
-    tile::cfft_pp<T, -1, NC, GP, NT, LS / 2>(reinterpret_cast<cx<T> *>(A),
+    tile::cfft_pp<T, -1, NC, GP, NT, LS / 2, OPQ>(reinterpret_cast<cx<T> *>(A),
                                             reinterpret_cast<cx<T> *>(B), W.tw);
-    if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false>(Z, Y, W.tq, sine);
-    else tile::post_fwd_pp<T, NC, GP, NT, LS>(Z, Y, kind, W.th, W.tq);
+    if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false, OPQ>(Z, Y, W.tq, sine);
+    else tile::post_fwd_pp<T, NC, GP, NT, LS, OPQ>(Z, Y, kind, W.th, W.tq);
     // forward elimination, plane by plane (dgtsv_homebrewed order)
 #pragma unroll
     for (int l = 0; l < GP; ++l) {
@@ -575,7 +576,7 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
       const double ak = a[k], bk = b[k], cc = c[k];
 #pragma unroll
       for (int u = 0; u < CPT; ++u) {
-        const int j = CPT * threadIdx.x + u;
+        const int j = CPT * tid + u;
         if (CPT * NT != n && j >= n) continue;
         const double y = (double)Y[l * LS + j];
         double pv;
@@ -650,7 +651,7 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
 }
 
 // ---------------------------------------------------------------- P3 -----
-template <typename T, int NC, int GP, int NT, bool PER>
+template <typename T, int NC, int GP, int NT, bool PER, bool OPQ>
 __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
                                             const double *__restrict__ ck,
                                             int nx, int nz, int nzs, int kind,
@@ -697,19 +698,19 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
   T pv[GP][CPT];
   double dck[CPT], q2ck[CPT];
   auto load = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
     // the recurrence restarts at the end of group g - 1 (unused, but read
     // in bounds, for g = 0); the checkpoint is issued first, so that the
     // factors can be recomputed while the lines are still arriving (loads
     // complete in issue order)
     const int c0 = max(g - 1, 0);
     const double *cg = ck + ((long long)i * nck + c0) * n;
-    load_cols<double, CPT, NT>(cg, dck, n);
-    if constexpr (PER) load_cols<double, CPT, NT>(cg + (long long)nx * nck * n, q2ck, n);
+    load_cols<double, CPT, NT>(cg, dck, n, tid);
+    if constexpr (PER) load_cols<double, CPT, NT>(cg + (long long)nx * nck * n, q2ck, n, tid);
     // branch-free: out-of-range planes/columns re-read valid entries
 #pragma unroll
     for (int l = 0; l < GP; ++l)
-      load_cols<T, CPT, NT>(line0 + (long long)min(k0 + l, nz - 1) * pstride, pv[l], n);
+      load_cols<T, CPT, NT>(line0 + (long long)min(k0 + l, nz - 1) * pstride, pv[l], n, tid);
   };
   // Stores of group g's lines (element pairs, 16-byte stores in FP64) from
   // R.  They are issued in the next group's step, after its loads have
@@ -718,11 +719,11 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
   // latency to it.
   constexpr int LD2 = (GP * n / 2 + NT - 1) / NT;
   auto flush = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
     const int np = min(GP, nz - k0);
 #pragma unroll
     for (int q = 0; q < LD2; ++q) {
-      const int t = threadIdx.x + q * NT;
+      const int t = tid + q * NT;
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       if (((GP * n / 2) % NT != 0 && t >= GP * n / 2) || l >= np) continue;
       V2 v;
@@ -739,9 +740,10 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
   for (int g = ngrp - 1; g >= 0; --g) {
     const int k0 = g * GP;
     const int np = min(GP, nz - k0);
+    const int tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int j = CPT * threadIdx.x + u;
+      const int j = CPT * tid + u;
       if (CPT * NT != n && j >= n) continue;
       // elimination factors of this group, recomputed from the checkpoint
       double d[GP], q2[GP];
@@ -829,7 +831,7 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
     }
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int j = CPT * threadIdx.x + u;
+      const int j = CPT * tid + u;
       if (CPT * NT != n && j >= n) continue;
       const int jp = d4 ? tile::d4_pos(j, n) : j;
       const bool neg = d4 && sine && (j & 1);
@@ -838,9 +840,9 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
     }
     __syncthreads();
     if (g > 0) load(g - 1);
-    if (d4) tile::d4_pre_pp<T, NC, GP, NT, LS, true>(A, B, W.th);
-    else tile::pre_inv_pp<T, NC, GP, NT, LS>(A, B, kind, W.th, W.tq);
-    tile::cfft_pp<T, +1, NC, GP, NT, LS / 2>(reinterpret_cast<cx<T> *>(B),
+    if (d4) tile::d4_pre_pp<T, NC, GP, NT, LS, true, OPQ>(A, B, W.th);
+    else tile::pre_inv_pp<T, NC, GP, NT, LS, OPQ>(A, B, kind, W.th, W.tq);
+    tile::cfft_pp<T, +1, NC, GP, NT, LS / 2, OPQ>(reinterpret_cast<cx<T> *>(B),
                                             reinterpret_cast<cx<T> *>(A), W.tw);
     if (d4) tile::d4_post<T, NC, GP, NT, LS, true>(R, W.tq, sine);
   }
@@ -870,6 +872,30 @@ template <typename T, int NC, bool PER>
 constexpr int slab_threads() {
   if (2 * NC != 512 && 2 * NC != 1024) return 256;
   return PER ? 256 : 512;
+}
+
+// Whether a single problem's slab pass computes its addresses anew in every
+// round (tile::lane_id): true where the registers they would hold keep a
+// workgroup from the CU that the LDS has room for, or push values into the
+// accumulation registers; false where the LDS or 512 threads set the residency
+// and the instructions only cost time.  Measured, addresses kept / computed
+// anew (us):
+//   FP64 P2, P3   200^3 periodic 61, 129 / 58, 70 (kept: one workgroup a CU);
+//                 192^3 62, 76 / 50, 54; 384x384x200 periodic P3 366 / 212;
+//                 400x800x200 509, 654 / 368, 402;
+//                 512^3 434, 453 / 491, 495; 400^3 P2 310 / 340
+//   FP32 P3       384^3 481 / 255, 768x768x256 1081 / 636 (its P2 keeps up only
+//                 so: 649 / 484), 400^3 570 / 361;
+//                 512^3 327 / 367; 1024x1024x128 periodic 805 / 532
+// A batch has workgroups of all lengths to fill a CU with and keeps its
+// addresses (64 problems 4547 / 4662).
+template <typename T, int NC, bool PER, bool BWD, bool CHUNK>
+constexpr bool slab_opaque() {
+  constexpr bool f32 = sizeof(T) == 4;
+  if (NC <= 160 || NC == 400 || (NC == 512 && f32 && PER)) return true;
+  if (!BWD) return f32 && (NC == 192 || NC == 384 || (NC == 200 && CHUNK) || (NC == 320 && PER));
+  if (NC == 384) return f32 || PER;
+  return NC == 192 || NC == 200 || NC == 320 || (NC == 1024 && f32);
 }
 
 // Threads of a batched slab workgroup (lines of up to 256 points): one

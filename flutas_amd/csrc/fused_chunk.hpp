@@ -142,7 +142,7 @@ __device__ __forceinline__ void zc_eliminate(const double *__restrict__ a,
 }
 
 // ---------------------------------------------------------------- P2 -----
-template <typename T, int NC, int GP, int NT, bool PER>
+template <typename T, int NC, int GP, int NT, bool PER, bool OPQ>
 __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, const ZChunks &zc,
                                              int nz, int msys, int kind,
                                              const double *__restrict__ lamx,
@@ -176,7 +176,7 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
   const double lx = lamx[i];
   double lam[CPT], dprev[CPT], pprev[CPT], w[CPT], S[CPT], E[CPT], ym[CPT];
   // d of the plane before the chunk (not used by the first chunk)
-  load_cols<double, CPT, NT>(zc.ckd + ((long long)i * zc.ngrp + gb) * n, dprev, n);
+  load_cols<double, CPT, NT>(zc.ckd + ((long long)i * zc.ngrp + gb) * n, dprev, n, threadIdx.x);
 #pragma unroll
   for (int u = 0; u < CPT; ++u) {
     const int j = CPT * threadIdx.x + u;
@@ -190,10 +190,10 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
   V2 r[LD];
   // branch-free prefetch; planes past the chunk (last group) re-read ke-1
   auto load = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int t = min((int)threadIdx.x + q * NT, GP * n / 2 - 1);
+      const int t = min(tid + q * NT, GP * n / 2 - 1);
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       r[q] = *reinterpret_cast<const V2 *>(line0 + (long long)min(k0 + l, ke - 1) * pstride + e);
     }
@@ -202,18 +202,19 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
   // (see yz_fwd_slab); hold[l] past the chunk repeats its last plane
   T hold[GP][CPT];
   auto flush = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int l = 0; l < GP; ++l)
-      store_cols_nt<T, CPT, NT>(line0 + (long long)min(k0 + l, ke - 1) * pstride, hold[l], n);
+      store_cols_nt<T, CPT, NT>(line0 + (long long)min(k0 + l, ke - 1) * pstride, hold[l], n, tid);
   };
   load(gb);
   for (int g = gb; g < ge; ++g) {
     const int k0 = g * GP;
     const int np = min(GP, ke - k0);
+    const int tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
-      const int t = threadIdx.x + q * NT;
+      const int t = tid + q * NT;
       if ((GP * n / 2) % NT != 0 && t >= GP * n / 2) continue;
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       const int p0 = trig ? (e >> 1) : e;
@@ -228,13 +229,13 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
       tile::d4_pre<T, NC, GP, NT, LS, false>(A, W.th);
       __syncthreads();
     }
-    tile::cfft_pp<T, -1, NC, GP, NT, LS / 2>(reinterpret_cast<cx<T> *>(A),
+    tile::cfft_pp<T, -1, NC, GP, NT, LS / 2, OPQ>(reinterpret_cast<cx<T> *>(A),
                                             reinterpret_cast<cx<T> *>(B), W.tw);
-    if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false>(Z, Y, W.tq, sine);
-    else tile::post_fwd_pp<T, NC, GP, NT, LS>(Z, Y, kind, W.th, W.tq);
+    if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false, OPQ>(Z, Y, W.tq, sine);
+    else tile::post_fwd_pp<T, NC, GP, NT, LS, OPQ>(Z, Y, kind, W.th, W.tq);
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int j = CPT * threadIdx.x + u;
+      const int j = CPT * tid + u;
       if (CPT * NT != n && j >= n) continue;
       T y[GP];
 #pragma unroll
@@ -248,9 +249,9 @@ __device__ __forceinline__ void yz_fwd_chunk(T *__restrict__ Wt, WStride ws, con
   }
   flush(ge - 1);
   double *sd = zc.side + ((long long)i * zc.nchunk + ch) * zc_side_slots(PER) * n;
-  store_cols<double, CPT, NT>(sd, E, n);
-  store_cols<double, CPT, NT>(sd + n, S, n);
-  if (PER && ch == zc.nchunk - 1) store_cols<double, CPT, NT>(sd + 2 * n, ym, n);
+  store_cols<double, CPT, NT>(sd, E, n, threadIdx.x);
+  store_cols<double, CPT, NT>(sd + n, S, n, threadIdx.x);
+  if (PER && ch == zc.nchunk - 1) store_cols<double, CPT, NT>(sd + 2 * n, ym, n, threadIdx.x);
 }
 
 // The reduced system of a slab's chunks, for the CPT columns of a thread (n
@@ -429,7 +430,7 @@ __device__ __forceinline__ void zc_substitute(const double *__restrict__ a,
 }
 
 // ---------------------------------------------------------------- P3 -----
-template <typename T, int NC, int GP, int NT, bool PER>
+template <typename T, int NC, int GP, int NT, bool PER, bool OPQ>
 __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, const ZChunks &zc,
                                              int nz, int msys, int kind,
                                              const double *__restrict__ lamx,
@@ -471,27 +472,27 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
   for (int u = 0; u < CPT; ++u) Pc[u] = pn[u] = pn2[u] = xm[u] = 0.0;
   zc_carries<CPT, PER>(
       zc, n, nch, i, ch, nz, a, b, c, pin, lam, Pc, pn, pn2, xm,
-      [](const double *line, double *v) { load_cols<double, CPT, NT>(line, v, n); });
+      [](const double *line, double *v) { load_cols<double, CPT, NT>(line, v, n, threadIdx.x); });
   T pv[GP][CPT];
   double dck[CPT], mck[CPT], qck[CPT];
   auto load = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
     // the group's starting values first (see zy_bwd_slab), then its lines
     const long long o = ((long long)i * zc.ngrp + g) * n;
-    load_cols<double, CPT, NT>(zc.ckd + o, dck, n);
-    load_cols<double, CPT, NT>(zc.ckm + o, mck, n);
-    if constexpr (PER) load_cols<double, CPT, NT>(zc.ckq + o, qck, n);
+    load_cols<double, CPT, NT>(zc.ckd + o, dck, n, tid);
+    load_cols<double, CPT, NT>(zc.ckm + o, mck, n, tid);
+    if constexpr (PER) load_cols<double, CPT, NT>(zc.ckq + o, qck, n, tid);
 #pragma unroll
     for (int l = 0; l < GP; ++l)
-      load_cols<T, CPT, NT>(line0 + (long long)min(k0 + l, ke - 1) * pstride, pv[l], n);
+      load_cols<T, CPT, NT>(line0 + (long long)min(k0 + l, ke - 1) * pstride, pv[l], n, tid);
   };
   constexpr int LD2 = (GP * n / 2 + NT - 1) / NT;
   auto flush = [&](int g) {
-    const int k0 = g * GP;
+    const int k0 = g * GP, tid = tile::lane_id<OPQ>();
     const int np = min(GP, ke - k0);
 #pragma unroll
     for (int q = 0; q < LD2; ++q) {
-      const int t = threadIdx.x + q * NT;
+      const int t = tid + q * NT;
       const int l = t / (n / 2), e = 2 * (t - l * (n / 2));
       if (((GP * n / 2) % NT != 0 && t >= GP * n / 2) || l >= np) continue;
       V2 v;
@@ -508,9 +509,10 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
   for (int g = ge - 1; g >= gb; --g) {
     const int k0 = g * GP;
     const int np = min(GP, ke - k0);
+    const int tid = tile::lane_id<OPQ>();
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int j = CPT * threadIdx.x + u;
+      const int j = CPT * tid + u;
       if (CPT * NT != n && j >= n) continue;
       zc_substitute<T, GP, PER>(
           a, b, c, k0, np, msys, pin, lam[u], dck[u], mck[u], PER ? qck[u] : 0.0, Pc[u], xm[u],
@@ -522,7 +524,7 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
     }
 #pragma unroll
     for (int u = 0; u < CPT; ++u) {
-      const int j = CPT * threadIdx.x + u;
+      const int j = CPT * tid + u;
       if (CPT * NT != n && j >= n) continue;
       const int jp = d4 ? tile::d4_pos(j, n) : j;
       const bool neg = d4 && sine && (j & 1);
@@ -531,9 +533,9 @@ __device__ __forceinline__ void zy_bwd_chunk(T *__restrict__ Wt, WStride ws, con
     }
     __syncthreads();
     if (g > gb) load(g - 1);
-    if (d4) tile::d4_pre_pp<T, NC, GP, NT, LS, true>(A, B, W.th);
-    else tile::pre_inv_pp<T, NC, GP, NT, LS>(A, B, kind, W.th, W.tq);
-    tile::cfft_pp<T, +1, NC, GP, NT, LS / 2>(reinterpret_cast<cx<T> *>(B),
+    if (d4) tile::d4_pre_pp<T, NC, GP, NT, LS, true, OPQ>(A, B, W.th);
+    else tile::pre_inv_pp<T, NC, GP, NT, LS, OPQ>(A, B, kind, W.th, W.tq);
+    tile::cfft_pp<T, +1, NC, GP, NT, LS / 2, OPQ>(reinterpret_cast<cx<T> *>(B),
                                             reinterpret_cast<cx<T> *>(A), W.tw);
     if (d4) tile::d4_post<T, NC, GP, NT, LS, true>(R, W.tq, sine);
   }

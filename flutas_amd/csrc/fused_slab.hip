@@ -13,8 +13,9 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
              const T *__restrict__ twh, const T *__restrict__ twq) {
   __shared__ __align__(16) T sm[2 * GP * line_stride<T, 2 * NC>()];
   __shared__ __align__(16) T stw[Tw<T, NC>::total];
-  yz_fwd_slab<T, NC, GP, NT, PER>(Wt, ws, ck, nx, nz, nzs, kind, lamx, lamy, a, b, c, pin, tw,
-                                  twh, twq, sm, stw, blockIdx.x);
+  constexpr bool OPQ = slab_opaque<T, NC, PER, false, false>();
+  yz_fwd_slab<T, NC, GP, NT, PER, OPQ>(Wt, ws, ck, nx, nz, nzs, kind, lamx, lamy, a, b, c, pin, tw,
+                                       twh, twq, sm, stw, blockIdx.x);
 }
 
 template <typename T, int NC, int GP, int NT, bool PER>
@@ -27,8 +28,9 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
              const T *__restrict__ twh, const T *__restrict__ twq) {
   __shared__ __align__(16) T sm[2 * GP * line_stride<T, 2 * NC>()];
   __shared__ __align__(16) T stw[Tw<T, NC>::total];
-  zy_bwd_slab<T, NC, GP, NT, PER>(Wt, ws, ck, nx, nz, nzs, kind, lamx, lamy, a, b, c, tw, twh,
-                                  twq, sm, stw, blockIdx.x);
+  constexpr bool OPQ = slab_opaque<T, NC, PER, true, false>();
+  zy_bwd_slab<T, NC, GP, NT, PER, OPQ>(Wt, ws, ck, nx, nz, nzs, kind, lamx, lamy, a, b, c, tw, twh,
+                                       twq, sm, stw, blockIdx.x);
 }
 
 template <typename T>

@@ -16,8 +16,9 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
   __shared__ __align__(16) T stw[Tw<T, NC>::total];
   int i, ch;
   zc_slab_of(nx, zc.nchunk, &i, &ch);
-  yz_fwd_chunk<T, NC, GP, NT, PER>(Wt, ws, zc, nz, msys, kind, lamx, lamy, a, b, c, pin, tw, twh,
-                                   twq, sm, stw, i, ch);
+  constexpr bool OPQ = slab_opaque<T, NC, PER, false, true>();
+  yz_fwd_chunk<T, NC, GP, NT, PER, OPQ>(Wt, ws, zc, nz, msys, kind, lamx, lamy, a, b, c, pin, tw,
+                                        twh, twq, sm, stw, i, ch);
 }
 
 template <typename T, int NC, int GP, int NT, bool PER>
@@ -31,8 +32,9 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
   __shared__ __align__(16) T stw[Tw<T, NC>::total];
   int i, ch;
   zc_slab_of(nx, zc.nchunk, &i, &ch);
-  zy_bwd_chunk<T, NC, GP, NT, PER>(Wt, ws, zc, nz, msys, kind, lamx, lamy, a, b, c, pin, tw, twh,
-                                   twq, sm, stw, i, ch);
+  constexpr bool OPQ = slab_opaque<T, NC, PER, true, true>();
+  zy_bwd_chunk<T, NC, GP, NT, PER, OPQ>(Wt, ws, zc, nz, msys, kind, lamx, lamy, a, b, c, pin, tw,
+                                        twh, twq, sm, stw, i, ch);
 }
 
 // Tables of the z-chunked passes, one thread per column (i, j), with the

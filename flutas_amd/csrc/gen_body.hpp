@@ -207,14 +207,6 @@ __device__ __forceinline__ void dftr(cx<T> *v) {
   else tile::dft<T, S, R>(v);
 }
 
-// The lane's index as a value the compiler knows nothing about: the LDS and
-// global addresses of every step are loop invariant, and kept in registers
-// across the loop over plane groups they cost a slab kernel 80 of them.
-__device__ __forceinline__ int lane_id() {
-  int t = threadIdx.x;
-  asm volatile("" : "+v"(t));
-  return t;
-}
 // Keeps the compiler from hoisting the LDS reads of all unrolled butterflies
 // and their twiddles to the front.
 __device__ __forceinline__ void read_fence() { asm volatile("" ::: "memory"); }
@@ -233,7 +225,7 @@ __device__ __forceinline__ void pass(cx<T> *buf, const cx<T> *tw, const Plan<T> 
   constexpr int PER = per_thread<EP, R>();
   const int nb = pl.N / R, ns = pl.ns[s], ts = pl.tstep[s];
   const unsigned nsm = pl.nsm[s];
-  const int tid = lane_id(), b0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), b0 = tid >> lgL, db = blockDim.x >> lgL;
   cx<T> *x = buf + (tid & ((1 << lgL) - 1)) * pl.lsc;
   cx<T> v[PER][R];
 #pragma unroll
@@ -276,7 +268,7 @@ template <typename T, int S, int EN>
 __device__ void pass_prime(cx<T> *buf, const cx<T> *tw, const Plan<T> &pl, int s, int lgL) {
   const int R = pl.radix[s], N = pl.N, nb = N / R, ns = pl.ns[s], ts = pl.tstep[s];
   const unsigned nsm = pl.nsm[s];
-  const int tid = lane_id(), o0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), o0 = tid >> lgL, db = blockDim.x >> lgL;
   cx<T> *x = buf + (tid & ((1 << lgL) - 1)) * pl.lsc;
   cx<T> acc[EN];
 #pragma unroll
@@ -350,7 +342,7 @@ __device__ __forceinline__ void post_fwd(T *sm, const Plan<T> &pl, KindBits kb,
                                          const Tables<T> &tb, int lgL) {
   constexpr int PER = EN / 2 + 1;
   const int N = pl.N, n = pl.n, np = N / 2 + 1;
-  const int tid = lane_id(), k0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), k0 = tid >> lgL, db = blockDim.x >> lgL;
   T *line = sm + (tid & ((1 << lgL) - 1)) * 2 * pl.lsc;
   const cx<T> *Z = reinterpret_cast<const cx<T> *>(line);
   T o[PER][4];
@@ -408,7 +400,7 @@ __device__ __forceinline__ void pre_inv(T *sm, const Plan<T> &pl, KindBits kb,
                                         const Tables<T> &tb, int lgL) {
   constexpr int PER = EN / 2 + 1;
   const int N = pl.N, n = pl.n, np = N / 2 + 1;
-  const int tid = lane_id(), k0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), k0 = tid >> lgL, db = blockDim.x >> lgL;
   T *line = sm + (tid & ((1 << lgL) - 1)) * 2 * pl.lsc;
   cx<T> z[PER][2];
 #pragma unroll
@@ -436,7 +428,7 @@ __device__ __forceinline__ void pre_inv(T *sm, const Plan<T> &pl, KindBits kb,
 // DCT-IV / DST-IV pre and post steps (tile::d4_pre, d4_post).
 template <typename T, bool CJ>
 __device__ __forceinline__ void d4_pre(T *sm, const Plan<T> &pl, const T *pre, int lgL) {
-  const int tid = lane_id(), k0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), k0 = tid >> lgL, db = blockDim.x >> lgL;
   cx<T> *Z = reinterpret_cast<cx<T> *>(sm) + (tid & ((1 << lgL) - 1)) * pl.lsc;
   for (int m = k0; m < pl.N; m += db) {
     const cx<T> v = tile::mul(Z[m], cx<T>{pre[2 * m], pre[2 * m + 1]});
@@ -448,7 +440,7 @@ template <typename T, int EN, bool CJ>
 __device__ __forceinline__ void d4_post(T *sm, const Plan<T> &pl, const T *post, bool sine,
                                         int lgL) {
   const int N = pl.N, n = pl.n;
-  const int tid = lane_id(), k0 = tid >> lgL, db = blockDim.x >> lgL;
+  const int tid = tile::lane_id<true>(), k0 = tid >> lgL, db = blockDim.x >> lgL;
   T *line = sm + (tid & ((1 << lgL) - 1)) * 2 * pl.lsc;
   const cx<T> *Z = reinterpret_cast<const cx<T> *>(line);
   T o[EN][2];
@@ -677,7 +669,7 @@ __device__ __forceinline__ void yz_fwd(T *__restrict__ Wt, WStride ws, const ZCh
   // branch free, entries past the group or the chunk repeat valid ones
   V2 r[LD];
   auto load = [&](int g) {
-    const int tid = lane_id();
+    const int tid = tile::lane_id<true>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
       const int t = min(tid + q * NT, GP * N - 1);
@@ -689,7 +681,7 @@ __device__ __forceinline__ void yz_fwd(T *__restrict__ Wt, WStride ws, const ZCh
   // yz_fwd_slab); hold[l] past the chunk repeats its last plane
   T hold[GP][CPT];
   auto flush = [&](int g) {
-    const int tid = lane_id();
+    const int tid = tile::lane_id<true>();
 #pragma unroll
     for (int l = 0; l < GP; ++l) {
       T *line = line0 + (long long)min(g * GP + l, ke - 1) * ws.wk;
@@ -700,7 +692,7 @@ __device__ __forceinline__ void yz_fwd(T *__restrict__ Wt, WStride ws, const ZCh
   };
   load(gb);
   for (int g = gb; g < ge; ++g) {
-    const int k0 = g * GP, np = min(GP, ke - k0), tid = lane_id();
+    const int k0 = g * GP, np = min(GP, ke - k0), tid = tile::lane_id<true>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
       const int t = tid + q * NT;
@@ -777,7 +769,7 @@ __device__ __forceinline__ void zy_bwd(T *__restrict__ Wt, WStride ws, const ZCh
   T pv[GP][CPT];
   double dck[CPT], mck[CPT], qck[CPT];
   auto load = [&](int g) {
-    const int tid = lane_id();
+    const int tid = tile::lane_id<true>();
     const long long o = ((long long)i * zc.ngrp + g) * n;
     get_cols<double, CPT>(zc.ckd + o, dck, n);
     get_cols<double, CPT>(zc.ckm + o, mck, n);
@@ -793,7 +785,7 @@ __device__ __forceinline__ void zy_bwd(T *__restrict__ Wt, WStride ws, const ZCh
     }
   };
   auto flush = [&](int g) {
-    const int k0 = g * GP, np = min(GP, ke - k0), tid = lane_id();
+    const int k0 = g * GP, np = min(GP, ke - k0), tid = tile::lane_id<true>();
 #pragma unroll
     for (int q = 0; q < LD; ++q) {
       const int t = tid + q * NT;

@@ -231,6 +231,18 @@ __device__ __forceinline__ cx<T> ptw(const T *__restrict__ tw, int rr, int j) {
   return w;
 }
 
+// The lane's index; OPQ: as a value the compiler knows nothing about.  The
+// LDS and global addresses of every step of a slab pass are loop invariant:
+// kept in registers across the loop over plane groups they cost 50 to 100 of
+// them, computed again in each round some 10% more instructions
+// (slab_opaque() says which is the better bargain).
+template <bool OPQ>
+__device__ __forceinline__ int lane_id() {
+  int t = threadIdx.x;
+  if constexpr (OPQ) asm volatile("" : "+v"(t));
+  return t;
+}
+
 // Stockham pass SI of radix R = Plan<N>::r[SI] over L lines (complex line
 // stride LSC), in place: all inputs are read into registers, then written.
 template <typename T, int S, int N, int SI, int L, int NT, int LSC>
@@ -328,14 +340,15 @@ __device__ __forceinline__ void d4_pre(T *sm, const T *__restrict__ pre) {
   }
 }
 // the same from src into dst, then a barrier
-template <typename T, int N, int L, int NT, int LS, bool CJ>
+template <typename T, int N, int L, int NT, int LS, bool CJ, bool OPQ = false>
 __device__ __forceinline__ void d4_pre_pp(const T *__restrict__ src, T *__restrict__ dst,
                                           const T *__restrict__ pre) {
   constexpr int TOT = L * N;
   constexpr int PER = (TOT + NT - 1) / NT;
+  const int tid = lane_id<OPQ>();
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int t = threadIdx.x + u * NT;
+    const int t = tid + u * NT;
     if (TOT % NT != 0 && t >= TOT) continue;
     const int l = t / N, m = t - (t / N) * N;
     const cx<T> *Z = reinterpret_cast<const cx<T> *>(src + l * LS);
@@ -385,14 +398,15 @@ __device__ __forceinline__ void d4_post(T *sm, const T *__restrict__ post, bool 
   __syncthreads();
 }
 // from src into dst, then a barrier
-template <typename T, int N, int L, int NT, int LS, bool CJ>
+template <typename T, int N, int L, int NT, int LS, bool CJ, bool OPQ = false>
 __device__ __forceinline__ void d4_post_pp(const T *__restrict__ src, T *__restrict__ dst,
                                            const T *__restrict__ post, bool sine) {
   constexpr int TOT = L * N;
   constexpr int PER = (TOT + NT - 1) / NT;
+  const int tid = lane_id<OPQ>();
 #pragma unroll 2
   for (int u = 0; u < PER; ++u) {
-    const int t = threadIdx.x + u * NT;
+    const int t = tid + u * NT;
     if (TOT % NT != 0 && t >= TOT) continue;
     const int l = t / N, k = t - (t / N) * N;
     const cx<T> W = reinterpret_cast<const cx<T> *>(src + l * LS)[k];
@@ -557,7 +571,7 @@ __device__ __forceinline__ void pre_inv(T *sm, int kind, const T *__restrict__ t
 // barrier at the end; no register staging (lower register pressure at the
 // cost of a second LDS tile).
 
-template <typename T, int S, int N, int SI, int L, int NT, int LSC>
+template <typename T, int S, int N, int SI, int L, int NT, int LSC, bool OPQ = false>
 __device__ __forceinline__ void pass_pp(const cx<T> *__restrict__ src, cx<T> *__restrict__ dst,
                                         const T *__restrict__ tw) {
   constexpr int R = Plan<N>::r[SI];
@@ -565,11 +579,12 @@ __device__ __forceinline__ void pass_pp(const cx<T> *__restrict__ src, cx<T> *__
   constexpr int NB = N / R;
   constexpr int TOT = L * NB;
   constexpr int PER = (TOT + NT - 1) / NT;
+  const int tid = lane_id<OPQ>();
   // fully unrolled over a thread's butterflies; src and dst never overlap,
   // so the reads of every butterfly can be issued before the first write
 #pragma unroll
   for (int u = 0; u < PER; ++u) {
-    const int t = threadIdx.x + u * NT;
+    const int t = tid + u * NT;
     if (TOT % NT != 0 && t >= TOT) continue;
     const int l = t / NB, b = t - (t / NB) * NB;
     const int j = b % NS;
@@ -592,28 +607,29 @@ __device__ __forceinline__ void pass_pp(const cx<T> *__restrict__ src, cx<T> *__
 
 // Complex FFT with ping-pong buffers: the result ends in `b` after an odd
 // number of passes (Plan<N>::nst), back in `a` after an even number.
-template <typename T, int S, int N, int L, int NT, int LSC>
+template <typename T, int S, int N, int L, int NT, int LSC, bool OPQ = false>
 __device__ __forceinline__ void cfft_pp(cx<T> *a, cx<T> *b, const T *__restrict__ tw) {
   using P = Plan<N>;
-  pass_pp<T, S, N, 0, L, NT, LSC>(a, b, tw);
-  if constexpr (P::nst > 1) pass_pp<T, S, N, 1, L, NT, LSC>(b, a, tw);
-  if constexpr (P::nst > 2) pass_pp<T, S, N, 2, L, NT, LSC>(a, b, tw);
+  pass_pp<T, S, N, 0, L, NT, LSC, OPQ>(a, b, tw);
+  if constexpr (P::nst > 1) pass_pp<T, S, N, 1, L, NT, LSC, OPQ>(b, a, tw);
+  if constexpr (P::nst > 2) pass_pp<T, S, N, 2, L, NT, LSC, OPQ>(a, b, tw);
 }
 
 // post_fwd from src (complex FFT of the packed lines) into dst.
-template <typename T, int N, int L, int NT, int LS>
+template <typename T, int N, int L, int NT, int LS, bool OPQ = false>
 __device__ __forceinline__ void post_fwd_pp(const T *__restrict__ src, T *__restrict__ dst,
                                             int kind, const T *__restrict__ twh,
                                             const T *__restrict__ twq) {
   constexpr int NP = N / 2 + 1;
   constexpr int TOT = L * NP;
   constexpr int PER = (TOT + NT - 1) / NT;
+  const int tid = lane_id<OPQ>();
   const bool trig = is_trig(kind), sine = is_sine(kind);
   // two items in flight per thread: their LDS reads overlap, at a bounded
   // register cost
 #pragma unroll 2
   for (int u = 0; u < PER; ++u) {
-    const int t = threadIdx.x + u * NT;
+    const int t = tid + u * NT;
     if (TOT % NT != 0 && t >= TOT) continue;
     const int l = t / NP, k = t - (t / NP) * NP;
     const cx<T> *Z = reinterpret_cast<const cx<T> *>(src + l * LS);
@@ -635,17 +651,18 @@ __device__ __forceinline__ void post_fwd_pp(const T *__restrict__ src, T *__rest
 }
 
 // pre_inv from src (real lines) into dst (complex Z').
-template <typename T, int N, int L, int NT, int LS>
+template <typename T, int N, int L, int NT, int LS, bool OPQ = false>
 __device__ __forceinline__ void pre_inv_pp(const T *__restrict__ src, T *__restrict__ dst,
                                            int kind, const T *__restrict__ twh,
                                            const T *__restrict__ twq) {
   constexpr int NP = N / 2 + 1;
   constexpr int TOT = L * NP;
   constexpr int PER = (TOT + NT - 1) / NT;
+  const int tid = lane_id<OPQ>();
   const bool trig = is_trig(kind), sine = is_sine(kind);
 #pragma unroll 2
   for (int u = 0; u < PER; ++u) {
-    const int t = threadIdx.x + u * NT;
+    const int t = tid + u * NT;
     if (TOT % NT != 0 && t >= TOT) continue;
     const int l = t / NP, k = t - (t / NP) * NP;
     const T *X = src + l * LS;
