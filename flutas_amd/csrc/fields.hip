@@ -10,6 +10,7 @@
 #include <atomic>
 #include <cmath>
 #include <mutex>
+#include <type_traits>
 #include <vector>
 
 namespace flutas {
@@ -28,6 +29,44 @@ __device__ __forceinline__ long long ixh(int i, int j, int k, int h, int nx,
 constexpr int kRowThreads = 1024;
 static inline dim3 grid3(int nx, int ny, int nz, int bx) {
   return dim3((nx + bx - 1) / bx, ny, nz);
+}
+
+// The workgroup's row: in grid order, or with XCD each of the 8 XCDs (which the
+// workgroups are dealt to round robin, each with its own L2) takes its eighth
+// of the rows in order, so that the rows j + 1 and k + 1 that a point reads
+// beside its own are found in that L2.  In grid order they are fetched once
+// per XCD, which bounds the passes whose fields stay in the 256 MB cache: FP64
+// 128^3 pres_tw_src 32.0 -> 24.2 us, correc 22.9 -> 19.2, correc_update_bc 31.2 ->
+// 27.2; 200x100x60 21.9 -> 15.7, 14.4 -> 12.3, 20.8 -> 18.8.  Where HBM bounds
+// them eighths of the field lose to grid order (192^3 pres_tw_src 110 -> 120 us;
+// 160^3 60 -> 44 alone, but a step of it 285 -> 290), and so does any split of
+// the passes that read little beside their row (256^3 fillps 95 -> 116).
+constexpr double kXcdBytes = 24e6;
+struct RowTile {
+  int i, j, k;
+};
+template <bool XCD>
+__device__ __forceinline__ RowTile row_tile() {
+  if constexpr (!XCD) {
+    return {(int)(blockIdx.x * blockDim.x + threadIdx.x) + 1, (int)blockIdx.y + 1,
+            (int)blockIdx.z + 1};
+  } else {
+    const unsigned gx = gridDim.x, gy = gridDim.y, per = gx * gy * gridDim.z >> 3;
+    const unsigned id = blockIdx.x + gx * (blockIdx.y + gy * blockIdx.z);
+    const unsigned L = id < 8 * per ? (id & 7) * per + (id >> 3) : id;
+    const unsigned row = L / gx, k = row / gy;
+    return {(int)((L - row * gx) * blockDim.x + threadIdx.x) + 1, (int)(row - k * gy) + 1,
+            (int)k + 1};
+  }
+}
+static inline bool rows_by_xcd(int nx, int ny, int nz, int elem_bytes) {
+  return (double)nx * ny * nz * elem_bytes <= kXcdBytes;
+}
+
+template <typename F>
+static inline void with_xcd(bool xcd, F f) {
+  if (xcd) f(std::true_type{});
+  else f(std::false_type{});
 }
 
 // ---- fillps (src/fillps.f90:42-61, _CONSTANT_COEFFS_POISSON) -------------
@@ -51,7 +90,7 @@ __global__ void __launch_bounds__(kRowThreads)
 }
 
 // ---- pres_tw_src (src/source.f90:272-306) -------------------------------
-template <typename T>
+template <typename T, bool XCD>
 __global__ void __launch_bounds__(kRowThreads)
     k_pres_tw_src(int nx, int ny, int nz, T dxi, T dyi, int nh_d,
                   int nh_u, const T *__restrict__ dzci, T rho0i,
@@ -60,8 +99,8 @@ __global__ void __launch_bounds__(kRowThreads)
                   const T *__restrict__ rho, T *__restrict__ u,
                   T *__restrict__ v, T *__restrict__ w, int cc) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y + 1, k = blockIdx.z + 1;
+  const RowTile rt = row_tile<XCD>();
+  const int i = rt.i, j = rt.j, k = rt.k;
   if (i > nx) return;
   const long long c1 = ixh(i, j, k, 1, nx, ny), cu = ixh(i, j, k, nh_u, nx, ny);
   const long long ip = c1 + 1, jp = c1 + (nx + 2),
@@ -108,7 +147,7 @@ __global__ void __launch_bounds__(kRowThreads)
 }
 
 // ---- correc (src/correc.f90:120-144) ------------------------------------
-template <typename T>
+template <typename T, bool XCD>
 __global__ void __launch_bounds__(kRowThreads)
     k_correc(int nx, int ny, int nz, int nh_d, int nh_u, T factori,
              T factorj, const T *__restrict__ dzci, T dt,
@@ -116,8 +155,8 @@ __global__ void __launch_bounds__(kRowThreads)
              T *__restrict__ v, T *__restrict__ w,
              const T *__restrict__ rho, int cc) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y + 1, k = blockIdx.z + 1;
+  const RowTile rt = row_tile<XCD>();
+  const int i = rt.i, j = rt.j, k = rt.k;
   if (i > nx) return;
   const long long c1 = ixh(i, j, k, 1, nx, ny), cu = ixh(i, j, k, nh_u, nx, ny);
   const long long ip = c1 + 1, jp = c1 + (nx + 2),
@@ -204,7 +243,7 @@ __device__ __forceinline__ double face_rule(char t, int side, double value, doub
   return factor + sgn * v;
 }
 
-template <bool BC>
+template <bool BC, bool XCD>
 __global__ void __launch_bounds__(kRowThreads)
     k_correc_update(int nx, int ny, int nz, int nh_d, int nh_u, double factori,
                     double factorj, const double *__restrict__ dzci, double dt,
@@ -213,8 +252,8 @@ __global__ void __launch_bounds__(kRowThreads)
                     double *__restrict__ v, double *__restrict__ w,
                     const double *__restrict__ rho, int cc, HaloBc hb) {
 #pragma clang fp contract(off)
-  const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-  const int j = blockIdx.y + 1, k = blockIdx.z + 1;
+  const RowTile rt = row_tile<XCD>();
+  const int i = rt.i, j = rt.j, k = rt.k;
   if (i > nx) return;
   const long long sy = nx + 2, sz = (long long)(nx + 2) * (ny + 2);
   const long long c1 = ixh(i, j, k, 1, nx, ny), cu = ixh(i, j, k, nh_u, nx, ny);
@@ -1205,10 +1244,12 @@ static int pres_tw_src_impl(int nx, int ny, int nz, T dxi, T dyi,
   if (!dzci || !p || !pold || !rho || !u || !v || !w) return fail(FLUTAS_EINVAL, "null pointer");
   const T f1 = T(1.0) + (f_t12 / f_t12_o), f2 = (f_t12 / f_t12_o);
   const int bx = xblock(nx);
-  hipLaunchKernelGGL(k_pres_tw_src<T>, grid3(nx, ny, nz, bx), dim3(bx), 0,
-                     current_stream(), nx, ny, nz, dxi, dyi, nh_d, nh_u, dzci,
-                     rho0i, f_t12, f1, f2, p, pold, rho, u, v, w,
-                     const_coeff ? 1 : 0);
+  with_xcd(rows_by_xcd(nx, ny, nz, sizeof(T)), [&](auto x) {
+    hipLaunchKernelGGL((k_pres_tw_src<T, x.value>), grid3(nx, ny, nz, bx), dim3(bx), 0,
+                       current_stream(), nx, ny, nz, dxi, dyi, nh_d, nh_u, dzci,
+                       rho0i, f_t12, f1, f2, p, pold, rho, u, v, w,
+                       const_coeff ? 1 : 0);
+  });
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }
@@ -1240,9 +1281,11 @@ static int correc_impl(int nx, int ny, int nz, int nh_d, int nh_u, T dxi,
     return fail(FLUTAS_EINVAL, "null pointer");
   const T rho0i = T(1.0) / rho0, factori = dt * dxi, factorj = dt * dyi;
   const int bx = xblock(nx);
-  hipLaunchKernelGGL(k_correc<T>, grid3(nx, ny, nz, bx), dim3(bx), 0,
-                     current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj,
-                     dzci, dt, rho0i, p, u, v, w, rho, const_coeff ? 1 : 0);
+  with_xcd(rows_by_xcd(nx, ny, nz, sizeof(T)), [&](auto x) {
+    hipLaunchKernelGGL((k_correc<T, x.value>), grid3(nx, ny, nz, bx), dim3(bx), 0,
+                       current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj,
+                       dzci, dt, rho0i, p, u, v, w, rho, const_coeff ? 1 : 0);
+  });
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }
@@ -1690,9 +1733,11 @@ int flutas_correc_update(int nx, int ny, int nz, int nh_d, int nh_u, double dxi,
   if (pnew == phi) return fail(FLUTAS_EINVAL, "pnew must not be the increment array phi");
   const double rho0i = 1.0 / rho0, factori = dt * dxi, factorj = dt * dyi;
   const int bx = xblock(nx);
-  hipLaunchKernelGGL(k_correc_update<false>, grid3(nx, ny, nz, bx), dim3(bx), 0,
-                     current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj, dzci, dt, rho0i,
-                     phi, pold, pnew, u, v, w, rho, const_coeff ? 1 : 0, HaloBc{});
+  with_xcd(rows_by_xcd(nx, ny, nz, 8), [&](auto x) {
+    hipLaunchKernelGGL((k_correc_update<false, x.value>), grid3(nx, ny, nz, bx), dim3(bx), 0,
+                       current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj, dzci, dt, rho0i,
+                       phi, pold, pnew, u, v, w, rho, const_coeff ? 1 : 0, HaloBc{});
+  });
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }
@@ -1733,9 +1778,11 @@ int flutas_correc_update_bc(int nx, int ny, int nz, int nh_d, int nh_u, double d
   hb.rank[2] = cbc[4] == 'P' ? 1 : 4;
   const double rho0i = 1.0 / rho0, factori = dt * dxi, factorj = dt * dyi;
   const int bx = xblock(nx);
-  hipLaunchKernelGGL(k_correc_update<true>, grid3(nx, ny, nz, bx), dim3(bx), 0,
-                     current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj, dzci, dt, rho0i,
-                     phi, pold, pnew, u, v, w, rho, const_coeff ? 1 : 0, hb);
+  with_xcd(rows_by_xcd(nx, ny, nz, 8), [&](auto x) {
+    hipLaunchKernelGGL((k_correc_update<true, x.value>), grid3(nx, ny, nz, bx), dim3(bx), 0,
+                       current_stream(), nx, ny, nz, nh_d, nh_u, factori, factorj, dzci, dt, rho0i,
+                       phi, pold, pnew, u, v, w, rho, const_coeff ? 1 : 0, hb);
+  });
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }
