@@ -15,6 +15,8 @@
 #include "internal.hpp"
 
 #include <cmath>
+#include <list>
+#include <mutex>
 
 namespace flutas {
 
@@ -490,32 +492,102 @@ int LineTables::build(int n_) {
     t4[2 * (N + 1) + 2 * m] = (double)cosl(b);
     t4[2 * (N + 1) + 2 * m + 1] = (double)-sinl(b);
   }
-  auto up = [](const std::vector<double> &h, double **dd, float **df) -> int {
-    FL_HIP(hipMalloc(dd, h.size() * sizeof(double)));
-    FL_HIP(hipMemcpy(*dd, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice));
-    std::vector<float> f(h.begin(), h.end());
-    FL_HIP(hipMalloc(df, f.size() * sizeof(float)));
-    FL_HIP(hipMemcpy(*df, f.data(), f.size() * sizeof(float), hipMemcpyHostToDevice));
-    return FLUTAS_OK;
-  };
-  FL_TRY(up(tw, &d_tw, &f_tw));
-  FL_TRY(up(twh, &d_twh, &f_twh));
-  FL_TRY(up(twq, &d_twq, &f_twq));
-  FL_TRY(up(twe, &d_twe, &f_twe));
-  FL_TRY(up(t4, &d_t4, &f_t4));
+  // one block and one copy: the FP64 tables, then their FP32 roundings, each
+  // from a 16-byte boundary (the counts are even)
+  const std::vector<double> *all[5] = {&tw, &twh, &twq, &twe, &t4};
+  size_t total = 0;
+  for (const auto *h : all) total += h->size();
+  std::vector<double> host(total + (total + 1) / 2 + 2 * 5);
+  float *hf = reinterpret_cast<float *>(host.data() + total);
+  FL_HIP(hipMalloc((void **)&mem, host.size() * sizeof(double)));
+  float *df = reinterpret_cast<float *>(mem + total);
+  double **dd[5] = {&d_tw, &d_twh, &d_twq, &d_twe, &d_t4};
+  float **ff[5] = {&f_tw, &f_twh, &f_twq, &f_twe, &f_t4};
+  size_t od = 0, of = 0;
+  for (int q = 0; q < 5; ++q) {
+    *dd[q] = mem + od;
+    *ff[q] = df + of;
+    for (size_t i = 0; i < all[q]->size(); ++i) {
+      host[od + i] = (*all[q])[i];
+      hf[of + i] = (float)(*all[q])[i];
+    }
+    od += all[q]->size();
+    of += (all[q]->size() + 3) & ~size_t(3);
+  }
+  FL_HIP(hipMemcpy(mem, host.data(), host.size() * sizeof(double), hipMemcpyHostToDevice));
   return FLUTAS_OK;
 }
 
 void LineTables::release() {
-  for (void *p : {(void *)d_tw, (void *)d_twh, (void *)d_twq, (void *)f_tw,
-                  (void *)f_twh, (void *)f_twq, (void *)d_ptw, (void *)f_ptw,
-                  (void *)d_twe, (void *)f_twe, (void *)d_t4, (void *)f_t4,
-                  (void *)d_gen, (void *)f_gen})
+  for (void *p : {(void *)mem, (void *)d_ptw, (void *)f_ptw, (void *)d_gen, (void *)f_gen})
     if (p) (void)hipFree(p);
-  d_tw = d_twh = d_twq = d_twe = d_t4 = nullptr;
+  mem = d_tw = d_twh = d_twq = d_twe = d_t4 = nullptr;
   f_tw = f_twh = f_twq = f_twe = f_t4 = nullptr;
   d_ptw = d_gen = nullptr;
   f_ptw = f_gen = nullptr;
+}
+
+// Tables of the stand-alone transforms, kept between calls as the plan of a
+// program that transforms the same lengths again (the reference makes its
+// FFTW plans once): tables built in each call cost it 340 us beside 70 us of
+// kernel (256 points).  The kTableLengths lengths used last stay, at most 0.9 MB
+// each; a caller holds its tables until its stream is done with them, so one
+// thread's eviction never takes another's.  clear_line_tables() gives them back.
+namespace {
+constexpr size_t kTableLengths = 16;
+struct KeptTables {
+  int dev, n;
+  std::shared_ptr<const LineTables> tab;
+};
+struct TableStore {
+  std::mutex mu;
+  std::list<KeptTables> kept;  // last used first
+};
+TableStore &table_store() {
+  // never destroyed: device memory cannot be freed after the runtime's own end
+  static TableStore *s = new TableStore;
+  return *s;
+}
+}  // namespace
+
+int line_tables(int n, std::shared_ptr<const LineTables> *out) {
+  int dev = 0;
+  FL_HIP(hipGetDevice(&dev));
+  TableStore &st = table_store();
+  auto find = [&] {
+    for (auto it = st.kept.begin(); it != st.kept.end(); ++it)
+      if (it->dev == dev && it->n == n) {
+        st.kept.splice(st.kept.begin(), st.kept, it);
+        *out = it->tab;
+        return true;
+      }
+    return false;
+  };
+  {
+    std::lock_guard<std::mutex> lk(st.mu);
+    if (find()) return FLUTAS_OK;
+  }
+  std::shared_ptr<LineTables> t(new LineTables, [](LineTables *p) {
+    p->release();
+    delete p;
+  });
+  FL_TRY(t->build(n));
+  std::shared_ptr<const LineTables> gone;  // freed after the lock
+  std::lock_guard<std::mutex> lk(st.mu);
+  if (find()) return FLUTAS_OK;  // another thread built it meanwhile
+  st.kept.push_front({dev, n, t});
+  if (st.kept.size() > kTableLengths) {
+    gone = st.kept.back().tab;
+    st.kept.pop_back();
+  }
+  *out = t;
+  return FLUTAS_OK;
+}
+
+void clear_line_tables() {
+  std::list<KeptTables> gone;
+  std::lock_guard<std::mutex> lk(table_store().mu);
+  gone.swap(table_store().kept);
 }
 
 template <typename T, typename Tin, typename Tout>

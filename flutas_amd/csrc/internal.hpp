@@ -6,6 +6,7 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -83,6 +84,7 @@ struct GenShape {
 struct LineTables {
   int n = 0, N = 0, nst = 0;
   int radix[kMaxStages] = {};
+  double *mem = nullptr;  // the block of the d_tw .. f_t4 tables
   double *d_tw = nullptr, *d_twh = nullptr, *d_twq = nullptr, *d_twe = nullptr;
   float *f_tw = nullptr, *f_twh = nullptr, *f_twq = nullptr, *f_twe = nullptr;
   double *d_t4 = nullptr;
@@ -101,6 +103,11 @@ struct LineTables {
   int build(int n);
   void release();
 };
+
+// The tables of n-point lines for a stand-alone transform on the current
+// device, from the kept ones or newly built (fft_lines.hip).
+int line_tables(int n, std::shared_ptr<const LineTables> *out);
+void clear_line_tables();
 
 // Geometry of a batch of lines: element e of line (l1,l2) lives at
 // base + l1*s1 + l2*s2 + e*se (separately for input and output).

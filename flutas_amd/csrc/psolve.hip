@@ -1131,15 +1131,14 @@ static int fft_guru_impl(int kind, int n, long long stride, int howmany1, long l
   // other kinds an even n
   if (kind != K_REDFT00 && kind != K_RODFT00 && (n & 1))
     return fail(FLUTAS_EINVAL, "line length must be even for this kind");
-  LineTables tab;
-  FL_TRY(tab.build(dft_length(kind, n)));
+  std::shared_ptr<const LineTables> tab;
+  FL_TRY(line_tables(dft_length(kind, n), &tab));
   LineGeom g;
   g.n = n; g.L1 = howmany1; g.L2 = howmany2;
   g.is1 = dist1; g.is2 = dist2; g.ise = stride;
   g.os1 = dist1; g.os2 = dist2; g.ose = stride;
-  int rc = launch_lines<T, T, T>(tab, kind, data, data, g, T(1), current_stream());
+  int rc = launch_lines<T, T, T>(*tab, kind, data, data, g, T(1), current_stream());
   hipError_t e = hipStreamSynchronize(current_stream());
-  tab.release();
   if (rc) return rc;
   if (e != hipSuccess) return fail(FLUTAS_EDEVICE, hipGetErrorString(e));
   return FLUTAS_OK;
@@ -1155,6 +1154,11 @@ int flutas_fft_guru(int kind, int n, long long stride, int howmany1, long long d
 int flutas_fft_guru_f32(int kind, int n, long long stride, int howmany1, long long dist1,
                         int howmany2, long long dist2, float *data) {
   return fft_guru_impl<float>(kind, n, stride, howmany1, dist1, howmany2, dist2, data);
+}
+
+int flutas_fft_cleanup(void) {
+  clear_line_tables();
+  return FLUTAS_OK;
 }
 
 int flutas_event_create(void **ev) {

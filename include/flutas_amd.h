@@ -249,6 +249,10 @@ int flutas_fft_lines(int kind, int n, int howmany, long long stride,
 int flutas_fft_guru(int kind, int n, long long stride, int howmany1,
                     long long dist1, int howmany2, long long dist2,
                     double *data);
+/* The tables of the 16 line lengths that flutas_fft_lines / _guru used last
+ * stay on the device between calls (as FFTW plans do); this gives them back,
+ * as fftw_cleanup. */
+int flutas_fft_cleanup(void);
 
 /* ---- batched solves (no counterpart in the reference, which solves one
  *      problem per call; for many independent small solves) ------------- */
