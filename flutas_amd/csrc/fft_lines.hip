@@ -530,7 +530,7 @@ void LineTables::release() {
 // Tables of the stand-alone transforms, kept between calls as the plan of a
 // program that transforms the same lengths again (the reference makes its
 // FFTW plans once): tables built in each call cost it 340 us beside 70 us of
-// kernel (256 points).  The kTableLengths lengths used last stay, at most 0.9 MB
+// kernel (256 points).  The kTableLengths lengths used last stay, at most 1.1 MB
 // each; a caller holds its tables until its stream is done with them, so one
 // thread's eviction never takes another's.  clear_line_tables() gives them back.
 namespace {
@@ -572,6 +572,8 @@ int line_tables(int n, std::shared_ptr<const LineTables> *out) {
     delete p;
   });
   FL_TRY(t->build(n));
+  if (fused_supported(n)) FL_TRY(build_fused_twiddles(*t));
+  else if (general_supported(n)) FL_TRY(add_general_tables(*t));
   std::shared_ptr<const LineTables> gone;  // freed after the lock
   std::lock_guard<std::mutex> lk(st.mu);
   if (find()) return FLUTAS_OK;  // another thread built it meanwhile

@@ -612,6 +612,78 @@ __device__ __forceinline__ void x_bwd(const T *__restrict__ Wt, WStride ws,
   }
 }
 
+// ---- stand-alone lines -----------------------------------------------------
+// In-place transform of L lines, numbered through both levels of the batch from
+// q0 on; lines of unit stride are loaded along themselves, others across the
+// lines.  base: L line offsets.
+template <typename T, bool FWD>
+__device__ __forceinline__ void lines(T *data, const LineGeom &g, int kind, const Plan<T> &pl,
+                                      int lgL, T *sm, long long *base, long long q0) {
+  const int n = pl.n, L = 1 << lgL, tot = n << lgL, NT = blockDim.x;
+  const int LS = 2 * pl.lsc;
+  const int nl = (int)min((long long)L, (long long)g.L1 * g.L2 - q0);
+  const KindBits kb = kind_bits(kind);
+  const bool along = g.ise == 1;
+  T *const stw = sm + L * LS;
+  if (threadIdx.x < L) {
+    // lines past the last repeat it
+    const long long q = q0 + min((int)threadIdx.x, nl - 1), l2 = q / g.L1;
+    base[threadIdx.x] = (q - l2 * g.L1) * g.is1 + l2 * g.is2;
+  }
+  cx<T> sr[kStage];
+  stage_load(sr, pl);
+  stage_store(sr, stw, pl);
+  const Tables<T> tb = tables(stw, pl);
+  __syncthreads();
+  auto line_of = [&](int t) { return along ? quot(t, pl.nm) : t & (L - 1); };
+  auto elem_of = [&](int t, int l) { return along ? t - l * n : t >> lgL; };
+  T r[2 * kXEN];
+#pragma unroll
+  for (int q = 0; q < 2 * kXEN; ++q) {
+    if (q * NT < tot) {
+      const int t = min((int)threadIdx.x + q * NT, tot - 1), l = line_of(t);
+      r[q] = data[base[l] + elem_of(t, l) * g.ise];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < 2 * kXEN; ++q) {
+    const int t = threadIdx.x + q * NT;
+    if (t < tot) {
+      const int l = line_of(t), e = elem_of(t, l);
+      T x = r[q];
+      int pos = e;
+      if (kb.d4) pos = tile::d4_pos(e, n);
+      else if (FWD && kb.trig) pos = tile::mk_pos(e, n);
+      if ((kb.d4 || (FWD && kb.trig)) && kb.sine && (e & 1)) x = -x;
+      sm[l * LS + pos] = x;
+    }
+  }
+  __syncthreads();
+  cx<T> *const buf = reinterpret_cast<cx<T> *>(sm);
+  if constexpr (FWD) {
+    if (kb.d4) d4_pre<T, false>(sm, pl, tb.th, lgL);
+    cfft<T, -1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+    if (kb.d4) d4_post<T, kXEN, false>(sm, pl, tb.tq, kb.sine, lgL);
+    else post_fwd<T, kXEN>(sm, pl, kb, tb, lgL);
+  } else {
+    pre_inv<T, kXEN>(sm, pl, kb, tb, lgL);
+    cfft<T, +1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+  }
+#pragma unroll 4
+  for (int t = threadIdx.x; t < tot; t += NT) {
+    const int l = line_of(t), e = elem_of(t, l);
+    if (l >= nl) continue;
+    int pos = e;
+    bool neg = false;
+    if (!FWD && kb.trig) {
+      pos = tile::mk_pos(e, n);
+      neg = kb.sine && (e & 1);
+    }
+    const T v = sm[l * LS + pos];
+    data[base[l] + e * g.ise] = neg ? -v : v;
+  }
+}
+
 // Columns of a thread: j = tid + u NT, u < CPT (whole waves of idle columns
 // skip the elimination).
 template <typename T, int CPT>

@@ -209,10 +209,13 @@ int general_group_planes(int ny) { return y_shape(ny).gp; }
 
 // The staged tables of the usual kinds, then those of REDFT11 / RODFT11.
 int build_general_tables(LineTables &tab, int n) {
-  const int N = n / 2;
   tab.release();
   tab.n = n;
-  tab.N = N;
+  tab.N = n / 2;
+  return add_general_tables(tab);
+}
+int add_general_tables(LineTables &tab) {
+  const int n = tab.n, N = tab.N;
   tab.gen_x[0] = x_shape(n, 8);
   tab.gen_x[1] = x_shape(n, 4);
   tab.gen_y = y_shape(n);
@@ -289,6 +292,39 @@ int launch_gen_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws, To
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }
+
+template <typename T, bool FWD>
+__global__ void __launch_bounds__(512)
+    k_g_lines(T *data, LineGeom g, int kind, gen::Plan<T> pl, int lgL) {
+  extern __shared__ __align__(16) unsigned char raw[];
+  __shared__ long long base[16];
+  gen::lines<T, FWD>(data, g, kind, pl, lgL, reinterpret_cast<T *>(raw), base,
+                     (long long)blockIdx.x << lgL);
+}
+bool gen_lines_supported(const LineTables &tab, int kind, long long lines) {
+  return tab.d_gen && kind != K_REDFT00 && kind != K_RODFT00 && lines <= 100000000LL;
+}
+template <typename T>
+int launch_gen_lines(const LineTables &tab, int kind, T *data, const LineGeom &g, hipStream_t s) {
+  const GenShape &x = tab.gen_x[sizeof(T) == 8 ? 0 : 1];
+  if (x.lgL < 0) return fail(FLUTAS_EUNSUPPORTED, "no tile for this length");
+  const gen::Plan<T> pl = gen_plan<T>(tab, x.rl, kind);
+  const int L = 1 << x.lgL;
+  const size_t lds = gen_lds(pl.N, L, sizeof(T));
+  const dim3 grid((unsigned)(((long long)g.L1 * g.L2 + L - 1) / L));
+  const bool fwd = kind != K_HC2R && kind != K_REDFT01 && kind != K_RODFT01;
+  if (fwd) {
+    FL_TRY(allow_lds(&k_g_lines<T, true>, lds));
+    hipLaunchKernelGGL((k_g_lines<T, true>), grid, dim3(x.nt), lds, s, data, g, kind, pl, x.lgL);
+  } else {
+    FL_TRY(allow_lds(&k_g_lines<T, false>, lds));
+    hipLaunchKernelGGL((k_g_lines<T, false>), grid, dim3(x.nt), lds, s, data, g, kind, pl, x.lgL);
+  }
+  FL_HIP(hipGetLastError());
+  return FLUTAS_OK;
+}
+template int launch_gen_lines<double>(const LineTables &, int, double *, const LineGeom &, hipStream_t);
+template int launch_gen_lines<float>(const LineTables &, int, float *, const LineGeom &, hipStream_t);
 
 // Calls f with the compile-time shape of a slab launch.
 template <int C, int G, bool P>

@@ -109,6 +109,18 @@ struct LineTables {
 int line_tables(int n, std::shared_ptr<const LineTables> *out);
 void clear_line_tables();
 
+// In-place transform of lines of a compiled length (lines.hip) and of the other
+// lengths of the four-pass pipeline (general.hip); the kinds and counts they
+// take.
+bool lines_tile_supported(const LineTables &tab, int kind, long long lines);
+template <typename T>
+int launch_lines_tile(const LineTables &tab, int kind, T *data, const struct LineGeom &g,
+                      hipStream_t s);
+bool gen_lines_supported(const LineTables &tab, int kind, long long lines);
+template <typename T>
+int launch_gen_lines(const LineTables &tab, int kind, T *data, const struct LineGeom &g,
+                     hipStream_t s);
+
 // Geometry of a batch of lines: element e of line (l1,l2) lives at
 // base + l1*s1 + l2*s2 + e*se (separately for input and output).
 struct LineGeom {
@@ -252,6 +264,7 @@ bool general_supported(int n);
 int general_group_planes(int ny);
 int general_slab_residency(int ny, int elem_bytes, int periodic, int *r2, int *r3);
 int build_general_tables(LineTables &tab, int n);
+int add_general_tables(LineTables &tab);  // beside those that build() made
 int gen_x_fwd_blocks(int n, int elem_bytes, int ny, int nz);
 template <typename T, typename Tin>
 int launch_gen_x_fwd(const LineTables &tx, int kind, const Tin *in, long long is1, long long is2,

@@ -1137,8 +1137,14 @@ static int fft_guru_impl(int kind, int n, long long stride, int howmany1, long l
   g.n = n; g.L1 = howmany1; g.L2 = howmany2;
   g.is1 = dist1; g.is2 = dist2; g.ise = stride;
   g.os1 = dist1; g.os2 = dist2; g.ose = stride;
-  int rc = launch_lines<T, T, T>(*tab, kind, data, data, g, T(1), current_stream());
-  hipError_t e = hipStreamSynchronize(current_stream());
+  const long long lines = (long long)howmany1 * howmany2;
+  hipStream_t s = current_stream();
+  int rc;
+  if (lines_tile_supported(*tab, kind, lines)) rc = launch_lines_tile<T>(*tab, kind, data, g, s);
+  else if (gen_lines_supported(*tab, kind, lines))
+    rc = launch_gen_lines<T>(*tab, kind, data, g, s);
+  else rc = launch_lines<T, T, T>(*tab, kind, data, data, g, T(1), s);
+  hipError_t e = hipStreamSynchronize(s);
   if (rc) return rc;
   if (e != hipSuccess) return fail(FLUTAS_EDEVICE, hipGetErrorString(e));
   return FLUTAS_OK;
