@@ -452,6 +452,28 @@ __host__ __device__ constexpr int checkpoints(int nz) {
   return (nz + GP - 1) / GP;
 }
 
+// The z coefficients of H rows that need no rule of their own (not the first
+// row, nor the last of the system or one past it), into scalar registers ahead of
+// the rows: without a branch between the rows what remains of an elimination is
+// the chain of its pivots.  Whole slabs, P2 and P3 (us): 512^3 periodic z 541, 626
+// -> 466, 532; 1024x1024x128 periodic z 864, 1060 -> 751, 886, its FP32 chain 718, 806
+// -> 447, 468; P2 of 1024x1024x512 2294 -> 2135; FP32 P3 of 512^3 331 -> 307.
+// Passes of 512 threads have 128 registers: there P2 of 512-point lines would spill
+// (441 -> 594) and the FP64 P3 loses (1024x1024x512 2335 -> 2655), so those keep
+// a branch per row.
+template <int H>
+__device__ __forceinline__ void slab_rows(const double *__restrict__ a,
+                                          const double *__restrict__ b,
+                                          const double *__restrict__ c, double *av, double *bv,
+                                          double *cv) {
+#pragma unroll
+  for (int l = 0; l < H; ++l) {
+    av[l] = a[l];
+    bv[l] = b[l];
+    cv[l] = c[l];
+  }
+}
+
 // The slab body (also used by the batched kernels): sm holds 2*GP lines
 // of line_stride<T, ny>() elements, stw the staged twiddles.
 template <typename T, int NC, int GP, int NT, bool PER, bool OPQ>
@@ -564,9 +586,41 @@ __device__ __forceinline__ void yz_fwd_slab(T *__restrict__ Wt, WStride ws,
                                             reinterpret_cast<cx<T> *>(B), W.tw);
     if (d4) tile::d4_post_pp<T, NC, GP, NT, LS, false, OPQ>(Z, Y, W.tq, sine);
     else tile::post_fwd_pp<T, NC, GP, NT, LS, OPQ>(Z, Y, kind, W.th, W.tq);
-    // forward elimination, plane by plane (dgtsv_homebrewed order)
+    // forward elimination, plane by plane (dgtsv_homebrewed order); a group of
+    // regular rows straight through (slab_rows)
+    constexpr bool STRAIGHT = PER || NT != 512 || NC != 256;
+    const bool regular = STRAIGHT && k0 > 0 && np == GP && k0 + GP < (PER ? nz - 1 : nzs);
+    if (regular) {
+      constexpr int H = GP < 8 ? GP : 8;
+#pragma unroll
+      for (int h = 0; h < GP; h += H) {
+        double av[H], bv[H], cv[H];
+        slab_rows<H>(a + k0 + h, b + k0 + h, c + k0 + h, av, bv, cv);
+#pragma unroll
+        for (int l = 0; l < H; ++l) {
+#pragma unroll
+          for (int u = 0; u < CPT; ++u) {
+            // columns past n repeat the last one and are not stored
+            const int j = min(CPT * tid + u, n - 1);
+            const double z = zrcp<T>((bv[l] + lam[u]) - av[l] * dprev[u]);
+            dprev[u] = cv[l] * z;
+            const double pv = ((double)Y[(h + l) * LS + j] - av[l] * pprev[u]) * z;
+            if constexpr (PER) {
+              const double q2 = (0.0 - av[l] * q2prev[u]) * z;
+              s1[u] = s1[u] + gk[u] * pv;
+              s2[u] = s2[u] + gk[u] * q2;
+              gk[u] = -(dprev[u] * gk[u]);
+              q2prev[u] = q2;
+            }
+            pprev[u] = pv;
+            hold[h + l][u] = (T)pv;
+          }
+        }
+      }
+    }
 #pragma unroll
     for (int l = 0; l < GP; ++l) {
+      if (regular) break;
       if (l >= np) {
 #pragma unroll
         for (int u = 0; u < CPT; ++u) hold[l][u] = hold[l - 1][u];
@@ -748,6 +802,42 @@ __device__ __forceinline__ void zy_bwd_slab(T *__restrict__ Wt, WStride ws,
       // elimination factors of this group, recomputed from the checkpoint
       double d[GP], q2[GP];
       double dp = dck[u];
+      // a group of regular rows straight through, see yz_fwd_slab
+      constexpr bool STRAIGHT = PER || NT != 512 || sizeof(T) == 4;
+      if (STRAIGHT && k0 > 0 && np == GP && k0 + GP < (PER ? nz - 1 : nzs)) {
+        constexpr int H = GP < 8 ? GP : 8;
+        double qp = PER ? q2ck[u] : 0.0;
+#pragma unroll
+        for (int h = 0; h < GP; h += H) {
+          double av[H], bv[H], cv[H];
+          slab_rows<H>(a + k0 + h, b + k0 + h, c + k0 + h, av, bv, cv);
+#pragma unroll
+          for (int l = 0; l < H; ++l) {
+            const double z = zrcp<T>((bv[l] + lam[u]) - av[l] * dp);
+            dp = cv[l] * z;
+            d[h + l] = dp;
+            if constexpr (PER) {
+              qp = (0.0 - av[l] * qp) * z;
+              q2[h + l] = qp;
+            }
+          }
+        }
+        double pn = pnext[u], pn2 = pnext2[u];
+#pragma unroll
+        for (int l = GP - 1; l >= 0; --l) {
+          const double p1 = (double)pv[l][u] - d[l] * pn;
+          pn = p1;
+          if constexpr (PER) {
+            pn2 = q2[l] - d[l] * pn2;
+            pv[l][u] = (T)(p1 + pn2 * plast[u]);
+          } else {
+            pv[l][u] = (T)p1;
+          }
+        }
+        pnext[u] = pn;
+        if constexpr (PER) pnext2[u] = pn2;
+        continue;
+      }
       if constexpr (!PER) {
 #pragma unroll
         for (int l = 0; l < GP; ++l) {
@@ -892,7 +982,7 @@ constexpr int slab_threads() {
 template <typename T, int NC, bool PER, bool BWD, bool CHUNK>
 constexpr bool slab_opaque() {
   constexpr bool f32 = sizeof(T) == 4;
-  if (NC <= 160 || NC == 400 || (NC == 512 && f32 && PER)) return true;
+  if (NC <= 160 || NC == 400 || ((NC == 512 || NC == 256) && f32 && PER)) return true;
   if (!BWD) return f32 && (NC == 192 || NC == 384 || (NC == 200 && CHUNK) || (NC == 320 && PER));
   if (NC == 384) return f32 || PER;
   return NC == 192 || NC == 200 || NC == 320 || (NC == 1024 && f32);
