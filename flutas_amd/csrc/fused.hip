@@ -42,7 +42,7 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
                                  xt.j0t * TJ, xt.k, nf_flag, nf_seq);
 }
 
-template <typename T, typename Tout, int NC, int TJ, int NT, bool ACC>
+template <typename T, typename Tout, int NC, int TJ, int NT, bool ACC, bool ALIGN>
 __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
     k_x_bwd(const T *__restrict__ Wt, WStride ws, Tout *__restrict__ out, long long os1,
             long long os2, int ny, int kind, T scale, const T *__restrict__ tw,
@@ -50,8 +50,8 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
   __shared__ __align__(16) T sm[TJ * line_stride<T, 2 * NC>()];
   __shared__ __align__(16) T stw[x_global_tw<T, NC>() ? 2 : Tw<T, NC>::total];
   const XTile xt = x_tile_of((ny + TJ - 1) / TJ);
-  x_bwd_tile<T, Tout, NC, TJ, NT, ACC>(Wt, ws, out, os1, os2, ny, kind, scale, tw, twh, twq, sm,
-                                       stw, xt.j0t * TJ, xt.k);
+  x_bwd_tile<T, Tout, NC, TJ, NT, ACC, ALIGN>(Wt, ws, out, os1, os2, ny, kind, scale, tw, twh,
+                                              twq, sm, stw, xt.j0t * TJ, xt.k);
 }
 
 // ---------------------------------------------------------------- host ---
@@ -120,6 +120,13 @@ int launch_x_fwd(const LineTables &tx, int kind, const Tin *in, long long is1,
   return FLUTAS_OK;
 }
 
+// FP64 outputs above this many bytes, in lines of 512 and 1024 points, are stored
+// from aligned lanes (x_bwd_tile): HBM takes whole memory lines sooner (P4 of 512^3
+// 462 -> 429 us, 1024x1024x512 2349 -> 2262), the cache does not mind and the
+// further lanes cost time (1024x256x128 137 -> 142 us, 512x512x160 143 -> 142; lines
+// of 640, 768 and 800 points 380 -> 406, 518 -> 554, 270 -> 289; FP32 transforms
+// 362 -> 376).
+constexpr double kAlignBytes = 512e6;
 template <typename T, typename Tout>
 int launch_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws,
                  Tout *out, long long os1, long long os2, int ny, int nz,
@@ -131,12 +138,19 @@ int launch_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws,
     constexpr int NT = tile_threads<T, NC>();
     constexpr int TJ = tile_lines<T, NC>();
     dim3 grid(((ny + TJ - 1) / TJ) * nz);
-    if (accumulate)
-      hipLaunchKernelGGL((k_x_bwd<T, Tout, NC, TJ, NT, true>), grid, dim3(NT), 0, s, Wt,
-                         ws, out, os1, os2, ny, kind, scale, pl.tw, th, tq);
-    else
-      hipLaunchKernelGGL((k_x_bwd<T, Tout, NC, TJ, NT, false>), grid, dim3(NT), 0, s, Wt,
-                         ws, out, os1, os2, ny, kind, scale, pl.tw, th, tq);
+    auto run = [&](auto kernel) {
+      hipLaunchKernelGGL(kernel, grid, dim3(NT), 0, s, Wt, ws, out, os1, os2, ny, kind, scale,
+                         pl.tw, th, tq);
+    };
+    if constexpr ((NC == 256 || NC == 512) && sizeof(T) == 8) {
+      if (!accumulate && (double)tx.n * ny * nz * sizeof(Tout) > kAlignBytes) {
+        run(&k_x_bwd<T, Tout, NC, TJ, NT, false, true>);
+        FL_HIP(hipGetLastError());
+        return FLUTAS_OK;
+      }
+    }
+    if (accumulate) run(&k_x_bwd<T, Tout, NC, TJ, NT, true, false>);
+    else run(&k_x_bwd<T, Tout, NC, TJ, NT, false, false>);
   });
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;

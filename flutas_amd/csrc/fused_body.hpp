@@ -272,7 +272,10 @@ __device__ __forceinline__ void x_fwd_tile(const Tin *__restrict__ in, long long
 
 // ---------------------------------------------------------------- P4 -----
 // Inverse of P1: out(i, j, k) = scale * r2r^-1 (x) (+ out when ACC).
-template <typename T, typename Tout, int NC, int TJ, int NT, bool ACC>
+// ALIGN: lanes start at the 128-byte boundary before a line of out, which the
+// halo puts anywhere, so that each wave stores whole memory lines; a line then
+// takes n and 128 bytes of lanes (kAlignBytes says where that pays).
+template <typename T, typename Tout, int NC, int TJ, int NT, bool ACC, bool ALIGN = false>
 __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
                                            Tout *__restrict__ out,
                                            long long os1, long long os2, int ny, int kind,
@@ -283,6 +286,13 @@ __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
   constexpr int n = 2 * NC;
   constexpr int LS = line_stride<T, n>();
   constexpr int LD = (TJ * n + NT - 1) / NT;
+  // lanes of a line of out and their elements
+  constexpr int AL = 128 / (int)sizeof(Tout), AW = ALIGN ? n + AL : n;
+  constexpr int LO = (TJ * AW + NT - 1) / NT;
+  auto elem = [](const Tout *row, int s) {
+    return ALIGN ? s - (int)((reinterpret_cast<unsigned long long>(row) / sizeof(Tout)) & (AL - 1))
+                 : s;
+  };
   const int nl = min(TJ, ny - j0);
   // d4: REDFT11 / RODFT11 (DCT-IV / DST-IV, tile_fft.hpp)
   const bool d4 = tile::is_d4(kind);
@@ -303,13 +313,14 @@ __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
   // (refined 1024x1024x512: this pass 3.34 -> 2.63 ms with 512 threads
   // against the preloading 256-thread form)
   constexpr bool LATE = ACC && NC == 512 && sizeof(T) == 4;
-  Tout prev[(ACC && !LATE) ? LD : 1];
+  Tout prev[(ACC && !LATE) ? LO : 1];
   if constexpr (ACC && !LATE) {
 #pragma unroll
-    for (int q = 0; q < LD; ++q) {
-      const int t = min((int)threadIdx.x + q * NT, TJ * n - 1);
-      const int l = t / n, e = t - (t / n) * n;
-      prev[q] = out[(long long)min(j0 + l, ny - 1) * os1 + (long long)k * os2 + e];
+    for (int q = 0; q < LO; ++q) {
+      const int t = min((int)threadIdx.x + q * NT, TJ * AW - 1);
+      const int l = t / AW;
+      const Tout *row = out + (long long)min(j0 + l, ny - 1) * os1 + (long long)k * os2;
+      prev[q] = row[max(0, min(elem(row, t - l * AW), n - 1))];
     }
   }
 #pragma unroll
@@ -338,10 +349,12 @@ __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
   tile::cfft<T, +1, NC, TJ, NT, LS / 2>(reinterpret_cast<cx<T> *>(sm), W.tw);
   if (d4) tile::d4_post<T, NC, TJ, NT, LS, true>(sm, W.tq, sine);
 #pragma unroll
-  for (int q = 0; q < LD; ++q) {
+  for (int q = 0; q < LO; ++q) {
     const int t = threadIdx.x + q * NT;
-    const int l = t / n, e = t - (t / n) * n;
-    if (t >= TJ * n || l >= nl) continue;
+    const int l = t / AW;
+    Tout *row = out + (long long)(j0 + l) * os1 + (long long)k * os2;
+    const int e = elem(row, t - l * AW);
+    if (t >= TJ * AW || l >= nl || (ALIGN && (e < 0 || e >= n))) continue;
     int pos = e;
     T sg = T(1);
     if (trig) {
@@ -349,7 +362,7 @@ __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
       if (sine && (e & 1)) sg = T(-1);
     }
     const T v = sm[l * LS + pos] * (scale * sg);
-    Tout *o = out + (long long)(j0 + l) * os1 + (long long)k * os2 + e;
+    Tout *o = row + e;
     if constexpr (LATE) *o = (Tout)((double)*o + (double)v);
     else if constexpr (ACC) *o = (Tout)((double)prev[q] + (double)v);
     else if constexpr (sizeof(T) == 8) st_nt((Tout)v, o);
