@@ -687,6 +687,15 @@ __global__ void __launch_bounds__(kRowThreads)
 // row reads as neighbours are then the rows its XCD's L2 is already
 // streaming.
 constexpr int kResidualPlanes = 32;
+// Grids of fewer than 8192 such walks take 8 planes a walk, so that the GPU's
+// slots fill (residual and check of 128^3 23, 22 -> 18, 14 us, 256^3 104, 82 -> 98, 82,
+// 400x300x200 182, 158 -> 169, 143; 512^3, 16384 walks, 727, 607 against 725, 627).
+constexpr int kResidualShort = 8;
+static int residual_planes(int nx, int ny, int nz) {
+  const long long walks = (long long)((nx + 255) / 256) * ny *
+                          ((nz + kResidualPlanes - 1) / kResidualPlanes);
+  return walks < 8192 ? kResidualShort : kResidualPlanes;
+}
 constexpr int kXcds = 8;
 
 struct BlockIdx3 {
@@ -711,7 +720,7 @@ struct Plane7 {
 
 // STORE: r receives the residual (held in registers through the walk);
 // without it only the maximum is formed, with no registers held.
-template <typename Tr, bool STORE>
+template <typename Tr, bool STORE, int KP>
 __global__ void __launch_bounds__(256)
     k_residual(OperatorDesc op, const double *__restrict__ f,
                const double *__restrict__ p, Tr *__restrict__ r,
@@ -722,8 +731,8 @@ __global__ void __launch_bounds__(256)
   const BlockIdx3 bi = residual_block(nbx, ny);
   const int i = bi.ib * blockDim.x + threadIdx.x;
   const int j = bi.j;
-  const int k0 = bi.kc * kResidualPlanes;
-  const int k1 = min(nz, k0 + kResidualPlanes);
+  const int k0 = bi.kc * KP;
+  const int k1 = min(nz, k0 + KP);
   const bool zper = op.cbc[4] == 'P';
   double am = 0.0;
   if (i < nx) {
@@ -762,7 +771,7 @@ __global__ void __launch_bounds__(256)
     Plane7 cur = gather(k0);
     Plane7 nxt = gather(knext(k0));
 #pragma unroll
-    for (int q = 0; q < kResidualPlanes; ++q) {
+    for (int q = 0; q < KP; ++q) {
       const int k = k0 + q;
       if (k >= k1) continue;
       Plane7 nxt2 = nxt;
@@ -903,15 +912,19 @@ template <typename Tr>
 int launch_residual(const OperatorDesc &op, const double *f, const double *p,
                     Tr *r, double *partial, int *nparts, hipStream_t s) {
   const int bx = 256;
-  const int nbx = (op.nx + bx - 1) / bx;
-  const long long nb = (long long)nbx * op.ny * ((op.nz + kResidualPlanes - 1) / kResidualPlanes);
+  const int nbx = (op.nx + bx - 1) / bx, kp = residual_planes(op.nx, op.ny, op.nz);
+  const long long nb = (long long)nbx * op.ny * ((op.nz + kp - 1) / kp);
   if (nb > 0x7fffffffLL) return fail(FLUTAS_EINVAL, "residual grid too large");
-  if (r)
-    hipLaunchKernelGGL((k_residual<Tr, true>), dim3((unsigned)nb), dim3(bx), 0, s, op, f, p, r,
-                       partial, nbx);
-  else
-    hipLaunchKernelGGL((k_residual<Tr, false>), dim3((unsigned)nb), dim3(bx), 0, s, op, f, p, r,
-                       partial, nbx);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)nb), dim3(bx), 0, s, op, f, p, r, partial, nbx);
+  };
+  if (kp == kResidualPlanes) {
+    if (r) run(&k_residual<Tr, true, kResidualPlanes>);
+    else run(&k_residual<Tr, false, kResidualPlanes>);
+  } else {
+    if (r) run(&k_residual<Tr, true, kResidualShort>);
+    else run(&k_residual<Tr, false, kResidualShort>);
+  }
   FL_HIP(hipGetLastError());
   *nparts = (int)nb;
   return FLUTAS_OK;
@@ -920,7 +933,8 @@ template int launch_residual<float>(const OperatorDesc &, const double *, const 
 template int launch_residual<double>(const OperatorDesc &, const double *, const double *, double *, double *, int *, hipStream_t);
 
 size_t residual_blocks(int nx, int ny, int nz) {
-  return (size_t)((nx + 255) / 256) * ny * ((nz + kResidualPlanes - 1) / kResidualPlanes);
+  const int kp = residual_planes(nx, ny, nz);
+  return (size_t)((nx + 255) / 256) * ny * ((nz + kp - 1) / kp);
 }
 
 int launch_absmax(const double *f, int nx, int ny, int nz, double *partial,
