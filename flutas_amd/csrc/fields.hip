@@ -869,7 +869,10 @@ int launch_accumulate(const float *r, double *p, int nx, int ny, int nz,
 
 // max over n partial maxima (NaN propagates), one workgroup
 __global__ void __launch_bounds__(1024)
-    k_reduce_max(const double *__restrict__ part, int n, double *__restrict__ out) {
+    k_reduce_max(const double *__restrict__ part0, int n0, const double *__restrict__ part1,
+                 int n1, double *__restrict__ out) {
+  const double *part = blockIdx.x ? part1 : part0;
+  const int n = blockIdx.x ? n1 : n0;
   __shared__ double wmax[16];
   double m[4] = {0.0, 0.0, 0.0, 0.0};
   auto take = [](double &acc, double o) {
@@ -896,12 +899,14 @@ __global__ void __launch_bounds__(1024)
   if (threadIdx.x == 0) {
     double r = wmax[0];
     for (int w = 1; w < 16; ++w) take(r, wmax[w]);
-    out[0] = r;
+    out[blockIdx.x] = r;
   }
 }
 
-int launch_reduce_max(const double *part, int n, double *out, hipStream_t s) {
-  hipLaunchKernelGGL(k_reduce_max, dim3(1), dim3(1024), 0, s, part, n, out);
+int launch_reduce_max(const double *part0, int n0, const double *part1, int n1, double *out,
+                      hipStream_t s) {
+  hipLaunchKernelGGL(k_reduce_max, dim3(n1 > 0 ? 2 : 1), dim3(1024), 0, s, part0, n0, part1, n1,
+                     out);
   FL_HIP(hipGetLastError());
   return FLUTAS_OK;
 }

@@ -378,6 +378,7 @@ int launch_flag_nonfinite(const double *f_halo, int nx, int ny, int nz, int *fla
 // partial count of launch_residual and launch_absmax
 size_t residual_blocks(int nx, int ny, int nz);
 // out[0] = max of n partial maxima (single workgroup)
-int launch_reduce_max(const double *part, int n, double *out, hipStream_t s);
+int launch_reduce_max(const double *part0, int n0, const double *part1, int n1, double *out,
+                      hipStream_t s);
 
 }  // namespace flutas
