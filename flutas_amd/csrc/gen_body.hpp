@@ -303,8 +303,9 @@ __device__ void pass_prime(cx<T> *buf, const cx<T> *tw, const Plan<T> &pl, int s
 }
 
 // Complex FFT of every line of the tile.  EP bounds a thread's butterflies
-// (see per_thread), EN its complex values.
-template <typename T, int S, int EP, int EN>
+// (see per_thread), EN its complex values; PRIME: the list may hold a prime
+// above 13 (its pass, a call, costs the kernel registers).
+template <typename T, int S, int EP, int EN, bool PRIME = true>
 __device__ __forceinline__ void cfft(cx<T> *buf, const cx<T> *tw, const Plan<T> &pl, int lgL) {
   for (int s = 0; s < pl.nst; ++s) {
     switch (pl.radix[s]) {
@@ -321,7 +322,9 @@ __device__ __forceinline__ void cfft(cx<T> *buf, const cx<T> *tw, const Plan<T> 
         if constexpr (EP >= 8) pass<T, S, EP, 13>(buf, tw, pl, s, lgL);
         else pass_prime<T, S, EN>(buf, tw, pl, s, lgL);
         break;
-      default: pass_prime<T, S, EN>(buf, tw, pl, s, lgL); break;
+      default:
+        if constexpr (PRIME) pass_prime<T, S, EN>(buf, tw, pl, s, lgL);
+        break;
     }
   }
 }
@@ -471,7 +474,7 @@ __device__ __forceinline__ void d4_post(T *sm, const Plan<T> &pl, const T *post,
 constexpr int kXEP = 8, kXEN = 16;
 
 // ---------------------------------------------------------------- P1 -----
-template <typename T, typename Tin>
+template <typename T, typename Tin, bool PRIME>
 __device__ __forceinline__ void x_fwd(const Tin *__restrict__ in, long long is1, long long is2,
                                       T *__restrict__ Wt, WStride ws, int ny, int kind,
                                       const Plan<T> &pl, int lgL, double *absmax_slot,
@@ -535,7 +538,7 @@ __device__ __forceinline__ void x_fwd(const Tin *__restrict__ in, long long is1,
   __syncthreads();
   cx<T> *const buf = reinterpret_cast<cx<T> *>(sm);
   if (kb.d4) d4_pre<T, false>(sm, pl, tb.th, lgL);
-  cfft<T, -1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+  cfft<T, -1, kXEP, kXEN, PRIME>(buf, tb.tw, pl, lgL);
   if (kb.d4) d4_post<T, kXEN, false>(sm, pl, tb.tq, kb.sine, lgL);
   else post_fwd<T, kXEN>(sm, pl, kb, tb, lgL);
   // transposed store: lanes along the lines
@@ -553,7 +556,7 @@ __device__ __forceinline__ void x_fwd(const Tin *__restrict__ in, long long is1,
 }
 
 // ---------------------------------------------------------------- P4 -----
-template <typename T, typename Tout, bool ACC>
+template <typename T, typename Tout, bool ACC, bool PRIME>
 __device__ __forceinline__ void x_bwd(const T *__restrict__ Wt, WStride ws,
                                       Tout *__restrict__ out, long long os1, long long os2,
                                       int ny, int kind, T scale, const Plan<T> &pl, int lgL,
@@ -592,7 +595,7 @@ __device__ __forceinline__ void x_bwd(const T *__restrict__ Wt, WStride ws,
   cx<T> *const buf = reinterpret_cast<cx<T> *>(sm);
   if (kb.d4) d4_pre<T, true>(sm, pl, tb.th, lgL);
   else pre_inv<T, kXEN>(sm, pl, kb, tb, lgL);
-  cfft<T, +1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+  cfft<T, +1, kXEP, kXEN, PRIME>(buf, tb.tw, pl, lgL);
   if (kb.d4) d4_post<T, kXEN, true>(sm, pl, tb.tq, kb.sine, lgL);
 #pragma unroll 4
   for (int t = threadIdx.x; t < tot; t += NT) {
@@ -616,7 +619,7 @@ __device__ __forceinline__ void x_bwd(const T *__restrict__ Wt, WStride ws,
 // In-place transform of L lines, numbered through both levels of the batch from
 // q0 on; lines of unit stride are loaded along themselves, others across the
 // lines.  base: L line offsets.
-template <typename T, bool FWD>
+template <typename T, bool FWD, bool PRIME>
 __device__ __forceinline__ void lines(T *data, const LineGeom &g, int kind, const Plan<T> &pl,
                                       int lgL, T *sm, long long *base, long long q0) {
   const int n = pl.n, L = 1 << lgL, tot = n << lgL, NT = blockDim.x;
@@ -662,12 +665,12 @@ __device__ __forceinline__ void lines(T *data, const LineGeom &g, int kind, cons
   cx<T> *const buf = reinterpret_cast<cx<T> *>(sm);
   if constexpr (FWD) {
     if (kb.d4) d4_pre<T, false>(sm, pl, tb.th, lgL);
-    cfft<T, -1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+    cfft<T, -1, kXEP, kXEN, PRIME>(buf, tb.tw, pl, lgL);
     if (kb.d4) d4_post<T, kXEN, false>(sm, pl, tb.tq, kb.sine, lgL);
     else post_fwd<T, kXEN>(sm, pl, kb, tb, lgL);
   } else {
     pre_inv<T, kXEN>(sm, pl, kb, tb, lgL);
-    cfft<T, +1, kXEP, kXEN>(buf, tb.tw, pl, lgL);
+    cfft<T, +1, kXEP, kXEN, PRIME>(buf, tb.tw, pl, lgL);
   }
 #pragma unroll 4
   for (int t = threadIdx.x; t < tot; t += NT) {

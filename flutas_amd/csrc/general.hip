@@ -25,27 +25,31 @@ __device__ __forceinline__ void gen_tile_of(int ntile, int *j0t, int *k) {
   *k = t / ntile;
 }
 
-template <typename T, typename Tin>
-__global__ void __launch_bounds__(512, 3)
+// The x and line kernels of lists without a prime above 13 hold two workgroups of
+// 512 threads per CU (128 registers); the pass of a prime wants more and those
+// lists keep kernels of their own (360x300x240 P1 201 us at 129 registers, 125 at
+// 102; 514 points, 257 a prime, 228 us, 292 with its registers cut).
+template <typename T, typename Tin, bool PRIME>
+__global__ void __launch_bounds__(512, PRIME ? 3 : 4)
     k_gx_fwd(const Tin *__restrict__ in, long long is1, long long is2, T *__restrict__ Wt,
              WStride ws, int ny, int kind, gen::Plan<T> pl, int lgL,
              double *__restrict__ absmax_part, int *nf_flag, int nf_seq) {
   extern __shared__ __align__(16) unsigned char gsm[];
   int j0t, k;
   gen_tile_of((ny + (1 << lgL) - 1) >> lgL, &j0t, &k);
-  gen::x_fwd<T, Tin>(in, is1, is2, Wt, ws, ny, kind, pl, lgL,
+  gen::x_fwd<T, Tin, PRIME>(in, is1, is2, Wt, ws, ny, kind, pl, lgL,
                      absmax_part ? absmax_part + blockIdx.x : nullptr, nf_flag, nf_seq,
                      reinterpret_cast<T *>(gsm), j0t << lgL, k);
 }
 
-template <typename T, typename Tout, bool ACC>
-__global__ void __launch_bounds__(512, 3)
+template <typename T, typename Tout, bool ACC, bool PRIME>
+__global__ void __launch_bounds__(512, PRIME ? 3 : 4)
     k_gx_bwd(const T *__restrict__ Wt, WStride ws, Tout *__restrict__ out, long long os1,
              long long os2, int ny, int kind, T scale, gen::Plan<T> pl, int lgL) {
   extern __shared__ __align__(16) unsigned char gsm[];
   int j0t, k;
   gen_tile_of((ny + (1 << lgL) - 1) >> lgL, &j0t, &k);
-  gen::x_bwd<T, Tout, ACC>(Wt, ws, out, os1, os2, ny, kind, scale, pl, lgL,
+  gen::x_bwd<T, Tout, ACC, PRIME>(Wt, ws, out, os1, os2, ny, kind, scale, pl, lgL,
                            reinterpret_cast<T *>(gsm), j0t << lgL, k);
 }
 
@@ -240,6 +244,12 @@ int add_general_tables(LineTables &tab) {
   return FLUTAS_OK;
 }
 
+static bool has_prime(const RadixList &rl) {
+  for (int q = 0; q < rl.nst; ++q)
+    if (rl.r[q] > 13) return true;
+  return false;
+}
+
 // Dynamic LDS beyond 64 KiB has to be asked for once per kernel.
 template <typename F>
 static int allow_lds(F *kernel, size_t bytes) {
@@ -258,11 +268,14 @@ int launch_gen_x_fwd(const LineTables &tx, int kind, const Tin *in, long long is
   const gen::Plan<T> pl = gen_plan<T>(tx, x.rl, kind);
   const int L = 1 << x.lgL;
   const size_t lds = gen_lds(pl.N, L, sizeof(T));
-  FL_TRY(allow_lds(&k_gx_fwd<T, Tin>, lds));
-  hipLaunchKernelGGL((k_gx_fwd<T, Tin>), dim3((ny + L - 1) / L * nz), dim3(x.nt), lds, s, in, is1,
-                     is2, Wt, ws, ny, kind, pl, x.lgL, absmax_part, nf_flag, nf_seq);
-  FL_HIP(hipGetLastError());
-  return FLUTAS_OK;
+  auto run = [&](auto kernel) -> int {
+    FL_TRY(allow_lds(kernel, lds));
+    hipLaunchKernelGGL(kernel, dim3((ny + L - 1) / L * nz), dim3(x.nt), lds, s, in, is1, is2, Wt,
+                       ws, ny, kind, pl, x.lgL, absmax_part, nf_flag, nf_seq);
+    FL_HIP(hipGetLastError());
+    return FLUTAS_OK;
+  };
+  return has_prime(x.rl) ? run(&k_gx_fwd<T, Tin, true>) : run(&k_gx_fwd<T, Tin, false>);
 }
 
 int gen_x_fwd_blocks(int n, int elem_bytes, int ny, int nz) {
@@ -280,25 +293,24 @@ int launch_gen_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws, To
   const int L = 1 << x.lgL;
   const size_t lds = gen_lds(pl.N, L, sizeof(T));
   const dim3 grid((ny + L - 1) / L * nz);
-  if (accumulate) {
-    FL_TRY((allow_lds(&k_gx_bwd<T, Tout, true>, lds)));
-    hipLaunchKernelGGL((k_gx_bwd<T, Tout, true>), grid, dim3(x.nt), lds, s, Wt, ws, out, os1, os2,
-                       ny, kind, scale, pl, x.lgL);
-  } else {
-    FL_TRY((allow_lds(&k_gx_bwd<T, Tout, false>, lds)));
-    hipLaunchKernelGGL((k_gx_bwd<T, Tout, false>), grid, dim3(x.nt), lds, s, Wt, ws, out, os1, os2,
-                       ny, kind, scale, pl, x.lgL);
-  }
-  FL_HIP(hipGetLastError());
-  return FLUTAS_OK;
+  auto run = [&](auto kernel) -> int {
+    FL_TRY(allow_lds(kernel, lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(x.nt), lds, s, Wt, ws, out, os1, os2, ny, kind, scale,
+                       pl, x.lgL);
+    FL_HIP(hipGetLastError());
+    return FLUTAS_OK;
+  };
+  if (has_prime(x.rl))
+    return accumulate ? run(&k_gx_bwd<T, Tout, true, true>) : run(&k_gx_bwd<T, Tout, false, true>);
+  return accumulate ? run(&k_gx_bwd<T, Tout, true, false>) : run(&k_gx_bwd<T, Tout, false, false>);
 }
 
-template <typename T, bool FWD>
-__global__ void __launch_bounds__(512)
+template <typename T, bool FWD, bool PRIME>
+__global__ void __launch_bounds__(512, PRIME ? 3 : 4)
     k_g_lines(T *data, LineGeom g, int kind, gen::Plan<T> pl, int lgL) {
   extern __shared__ __align__(16) unsigned char raw[];
   __shared__ long long base[16];
-  gen::lines<T, FWD>(data, g, kind, pl, lgL, reinterpret_cast<T *>(raw), base,
+  gen::lines<T, FWD, PRIME>(data, g, kind, pl, lgL, reinterpret_cast<T *>(raw), base,
                      (long long)blockIdx.x << lgL);
 }
 bool gen_lines_supported(const LineTables &tab, int kind, long long lines) {
@@ -313,15 +325,14 @@ int launch_gen_lines(const LineTables &tab, int kind, T *data, const LineGeom &g
   const size_t lds = gen_lds(pl.N, L, sizeof(T));
   const dim3 grid((unsigned)(((long long)g.L1 * g.L2 + L - 1) / L));
   const bool fwd = kind != K_HC2R && kind != K_REDFT01 && kind != K_RODFT01;
-  if (fwd) {
-    FL_TRY(allow_lds(&k_g_lines<T, true>, lds));
-    hipLaunchKernelGGL((k_g_lines<T, true>), grid, dim3(x.nt), lds, s, data, g, kind, pl, x.lgL);
-  } else {
-    FL_TRY(allow_lds(&k_g_lines<T, false>, lds));
-    hipLaunchKernelGGL((k_g_lines<T, false>), grid, dim3(x.nt), lds, s, data, g, kind, pl, x.lgL);
-  }
-  FL_HIP(hipGetLastError());
-  return FLUTAS_OK;
+  auto run = [&](auto kernel) -> int {
+    FL_TRY(allow_lds(kernel, lds));
+    hipLaunchKernelGGL(kernel, grid, dim3(x.nt), lds, s, data, g, kind, pl, x.lgL);
+    FL_HIP(hipGetLastError());
+    return FLUTAS_OK;
+  };
+  if (has_prime(x.rl)) return fwd ? run(&k_g_lines<T, true, true>) : run(&k_g_lines<T, false, true>);
+  return fwd ? run(&k_g_lines<T, true, false>) : run(&k_g_lines<T, false, false>);
 }
 template int launch_gen_lines<double>(const LineTables &, int, double *, const LineGeom &, hipStream_t);
 template int launch_gen_lines<float>(const LineTables &, int, float *, const LineGeom &, hipStream_t);
