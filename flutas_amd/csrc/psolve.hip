@@ -404,15 +404,15 @@ int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
 // unpenalised score took 6, the penalised one takes 2; refined 128^3:
 // 0.309, 0.244, 0.230, 0.207, 0.249, 0.225 ms, 4 either way).
 // Measured FP64 solves (ms for 1/2/3/4/6/8 chunks; * the count taken):
-//   768x768x256 NN-z      2.81  2.69* 2.72  2.71  2.79  2.79
-//   640x640x320 NN-z      2.85  2.55  2.56  2.49* 2.59  2.57
-//   640x640x256 periodic  2.49  2.13  2.14  2.10* 2.17  2.18
-//   384x768x256 DD-z      1.54  1.38  1.42  1.32* 1.38  1.38
-//   512^3 NN-z            1.92* 1.90  1.92  1.98  1.96  1.95
-//   1024x1024x512 NN-z    9.68* 10.0  10.1  10.1  10.3  10.5
-//   256x256x512 periodic  0.78  0.55* 0.63  0.61  0.62  0.60
-//   400^3 NN-z            1.26  1.23  1.15  1.19  1.16  1.21  (5 taken)
-// and at 128^3: 0.115, 0.082 (2), 0.065 (4, taken), 0.072 (8).
+//   768x768x256 NN-z      2.71  2.65* 2.68  2.67  2.75  2.76
+//   640x640x320 NN-z      2.65  2.46  2.48  2.42* 2.51  2.50
+//   640x640x256 periodic  2.24  2.02  2.06  2.01* 2.07  2.10
+//   384x768x256 DD-z      1.41  1.36  1.39  1.28* 1.34  1.33
+//   512^3 NN-z            1.69* 1.71  1.71  1.81  1.75  1.77
+//   1024x1024x512 NN-z    8.77* 9.47  9.46  9.56  9.68  9.76
+//   256x256x512 periodic  0.70  0.53* 0.56  0.59  0.57  0.57
+//   400^3 NN-z            1.09  1.18  1.10  1.13  1.13  1.16  (5 taken: 1.06)
+// and at 128^3: 0.114, 0.082 (2), 0.069 (4, taken), 0.078 (8).
 int default_zchunks(const flutas_psolve *h, int elem) {
   if (!h->fused) return 1;
   const int per = (h->cbc[4] == 'P');

@@ -138,7 +138,8 @@ const char *flutas_psolve_stage_name(const flutas_psolve *h, int stage);
  * z elimination, 2 z substitution and y backward, 3 x backward) launched
  * `reps` (<= 16) times back to back after one solve f -> p: *ms = the
  * average duration of one launch, from two HIP events on the library
- * stream.  The work field is left transformed; p holds the solution. */
+ * stream.  The work field is left transformed; p holds the solution.
+ * Plans with both lengths compiled; EUNSUPPORTED for the others. */
 int flutas_psolve_time_stage(flutas_psolve *h, const double *f, double *p, int stage,
                              int reps, double *ms);
 
@@ -148,9 +149,10 @@ int flutas_psolve_time_stage(flutas_psolve *h, const double *f, double *p, int s
  * n chunks (1..8) by separate workgroups and joined by a reduced system of
  * two unknowns per chunk and column, which gives plans with few x-slabs
  * more workgroups than the GPU has CUs.  n = 0 restores the plan's default
- * (the count, with chunks of 32 planes or more, that best fills the GPU's
- * workgroup slots over the two slab passes, from the CU count and the
- * kernels' occupancy); n = 1 walks whole slabs.  The count may come out lower than n for
+ * (the count that best fills the GPU's workgroup slots over the two slab
+ * passes, from the CU count and the kernels' occupancy, with chunks of 32
+ * planes or more unless the workgroups do not reach the CUs); n = 1 walks
+ * whole slabs.  FP32 solves on an FP64 plan follow n, or their own default.  The count may come out lower than n for
  * a short z.  Results equal the whole-slab walk's to rounding; the pivots
  * stay the reference's bit for bit.  Changing the count frees the tables a
  * recorded graph of this plan's solve refers to: record again after it.
