@@ -572,7 +572,7 @@ int solve_f32(flutas_psolve *h, const float *f, float *p, hipStream_t s) {
   const Geo q = halo_geo(h);
   ++h->seq;
   FL_TRY((spectral<float, float, float>(h, f + q.interior, true, p + q.interior, 0, h->W32, s,
-                                        nullptr, h->compiled() ? h->nf_dev : nullptr)));
+                                        nullptr, h->fused ? h->nf_dev : nullptr)));
   h->last_iters = 0;
   h->last_relres = -1.0;
   return FLUTAS_OK;
@@ -923,7 +923,7 @@ int flutas_psolve_solve_f32(flutas_psolve *h, float *p) {
   hipStream_t s = current_stream();
   FL_TRY(solve_f32(h, p, p, s));
   FL_HIP(hipStreamSynchronize(s));
-  if (h->compiled() && *(volatile int *)h->nf_host == h->seq)
+  if (h->fused && *(volatile int *)h->nf_host == h->seq)
     return fail(FLUTAS_ENONFINITE, "right-hand side holds NaN or Inf");
   return FLUTAS_OK;
 }

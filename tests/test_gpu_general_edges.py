@@ -1,0 +1,34 @@
+"""Line lengths without a compiled plan at the edges of what the other tests
+cover: non-finite FP32 fields, with the general kernels in x, in y and in
+both."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from cases import z_metrics
+
+pytestmark = pytest.mark.gpu
+
+
+def _solve32(api, plan, d):
+    return api.lib.flutas_psolve_solve_f32(C.c_void_p(plan._h),
+                                           C.cast(C.c_void_p(d.ptr), C.POINTER(C.c_float)))
+
+
+@pytest.mark.parametrize("bad", [np.nan, np.inf])
+@pytest.mark.parametrize("ng", [(36, 64, 20), (64, 300, 20), (90, 154, 20), (64, 32, 20)])
+def test_f32_nonfinite_is_reported(api, oracle, ng, bad):
+    """As flutas_psolve_solve_f32 states for the four-pass pipeline; a field
+    without it solves on the same plan before and after."""
+    _, _, dzci, dzfi, _, _ = z_metrics(oracle, ng[2], 0.0, 1.0)
+    plan = api.PoissonPlan(ng, tuple(float(n) for n in ng), dzci, dzfi, "PPDDNN")
+    f = np.zeros(tuple(n + 2 for n in ng), np.float32, order="F")
+    f[1:-1, 1:-1, 1:-1] = np.random.default_rng(1).standard_normal(ng)
+    g = f.copy(order="F")
+    g[5, 7, 4] = bad
+    for field, code in ((f, 0), (g, api.FLUTAS_ENONFINITE), (f, 0)):
+        d = api.DeviceArray.from_host(field)
+        assert _solve32(api, plan, d) == code
+        assert np.all(np.isfinite(d.to_host())) == (code == 0)
+    plan.destroy()
