@@ -312,6 +312,7 @@ const ChunkSet &chunks_of(const flutas_psolve *h) {
 template <typename T>
 int slab_fwd(flutas_psolve *h, T *W, WStride ws, int pin, int per, hipStream_t s) {
   const ChunkSet &z = chunks_of<T>(h);
+  if (h->gy && !z.mem) return fail(FLUTAS_ENOMEM, "the plan has no z chunk tables");
   if (h->gy)
     return launch_gen_yz_fwd<T>(h->ty, h->kinds[2], W, ws, z.zc, h->nx, h->nz,
                                 per ? h->nz - 1 : h->nzs, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
@@ -370,11 +371,11 @@ int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
   const int ngrp = (nz + gp - 1) / gp;
   const size_t nd = zchunk_doubles(h->nx, h->ny, ngrp, nch, per != 0);
   FL_HIP(hipMalloc((void **)&z.mem, nd * sizeof(double)));
-  const int rc = build_zchunk_tables(z.mem, &z.zc, h->nx, h->ny, nz, per ? nz - 1 : h->nzs, gp,
-                                     cpl, nch, per != 0, pin, elem, h->d_lamx, h->d_lamy, h->d_a,
-                                     h->d_b, h->d_c, nullptr);
+  int rc = build_zchunk_tables(z.mem, &z.zc, h->nx, h->ny, nz, per ? nz - 1 : h->nzs, gp, cpl, nch,
+                               per != 0, pin, elem, h->d_lamx, h->d_lamy, h->d_a, h->d_b, h->d_c,
+                               nullptr);
   if (rc == FLUTAS_OK && hipDeviceSynchronize() != hipSuccess)
-    return fail(FLUTAS_EDEVICE, "z chunk tables");
+    rc = fail(FLUTAS_EDEVICE, "z chunk tables");
   if (rc) {
     (void)hipFree(z.mem);
     z = ChunkSet{};
@@ -465,18 +466,27 @@ void build_chunks32(flutas_psolve *h) {
 int plan_elem(const flutas_psolve *h) { return h->precision == FLUTAS_FP64 ? 8 : 4; }
 
 // The chunk count of the plan: n for its own chain; the tables of solve_f32
-// follow zreq where they were made.
+// follow zreq where they were made.  The old tables make room for the new
+// ones; where those cannot be made the plan goes back to the count it had (a
+// general y length has no pass without tables).
 int set_zchunks(flutas_psolve *h, int n) {
   if (n < 1 || n > kMaxZChunks) return fail(FLUTAS_EINVAL, "z chunks must be 1..8");
+  const int before = h->zcs.n;
   if (h->zcs.mem || h->zcs32.mem) {
     FL_HIP(hipDeviceSynchronize());
     (void)hipFree(h->zcs.mem);
     (void)hipFree(h->zcs32.mem);
     h->zcs = h->zcs32 = ChunkSet{};
   }
-  FL_TRY(build_chunks(h, h->zcs, plan_elem(h), n));
+  const int rc = build_chunks(h, h->zcs, plan_elem(h), n);
+  if (rc) {
+    (void)hipGetLastError();
+    const std::string why = flutas_last_error();
+    (void)build_chunks(h, h->zcs, plan_elem(h), before);
+    set_error(why);
+  }
   if (h->has32) build_chunks32(h);
-  return FLUTAS_OK;
+  return rc;
 }
 
 // One spectral solve in storage/arithmetic T: the right-hand side `in`
@@ -1190,8 +1200,11 @@ int flutas_event_destroy(void *ev) {
 int flutas_psolve_set_zchunks(flutas_psolve *h, int n) {
   if (!h) return fail(FLUTAS_EINVAL, "null plan");
   if (n < 0 || n > kMaxZChunks) return fail(FLUTAS_EINVAL, "z chunks must be 1..8");
+  const int before = h->zreq;
   h->zreq = n;
-  return set_zchunks(h, n == 0 ? default_zchunks(h, plan_elem(h)) : n);
+  const int rc = set_zchunks(h, n == 0 ? default_zchunks(h, plan_elem(h)) : n);
+  if (rc) h->zreq = before;
+  return rc;
 }
 
 int flutas_psolve_zchunks(const flutas_psolve *h, int *n) {

@@ -1,0 +1,50 @@
+"""What the host side of the library allocates, launches and waits for, and what
+it does when device memory is short, on the CPU: the library over a stand-in
+for the HIP runtime that records launches and bounds the memory."""
+import pytest
+
+import hipsim
+
+
+# FP64 and refined plans whose y lines run the general kernels
+@pytest.mark.parametrize("ng,kw", [((90, 300, 60), "{}"), ((64, 154, 60), "dict(precision=32)")])
+def test_plan_survives_a_chunk_count_that_does_not_fit(tmp_path, ng, kw):
+    hipsim.run(f"""
+ng = {ng}
+p = plan(ng, **{kw})
+f, g = field(ng), field(ng)
+first = p.set_zchunks(2)
+assert first == 2
+d32 = field(ng, np.float32)
+assert solve32(p, d32) == 0
+used = sim.sim_used()
+
+def solves():
+    sim.sim_reset()
+    rc = api.lib.flutas_psolve_solve_into(C.c_void_p(p._h), f.c, g.c)
+    assert sim.sim_count(2) == 0, "a launch was refused"
+    return rc, [l[0] for l in launches()]
+
+rc, names = solves()
+assert rc in (0, api.FLUTAS_ENOTCONV), rc
+# room for what there is and nothing more
+sim.sim_limit(used)
+for call in (lambda: p.set_zchunks(8), lambda: p.tune(f, g, 1)):
+    try:
+        call()
+        raise SystemExit("tables beyond the memory")
+    except api.FlutasError as e:
+        assert "memory" in str(e), e
+    n = C.c_int()
+    api.lib.flutas_psolve_zchunks(C.c_void_p(p._h), C.byref(n))
+    assert 1 <= n.value <= 2
+    assert solves()[0] == rc
+    assert solve32(p, d32) == 0 and sim.sim_count(2) == 0
+sim.sim_limit(UNLIMITED)
+assert p.set_zchunks(8) > 2
+assert solves() == (rc, names)
+assert solve32(p, d32) == 0
+p.destroy(); f.free(); g.free(); d32.free()
+api.lib.flutas_fft_cleanup()
+assert sim.sim_used() == 0, "device memory left"
+""", tmp_path)
