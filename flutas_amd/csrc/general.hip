@@ -250,12 +250,15 @@ static bool has_prime(const RadixList &rl) {
   return false;
 }
 
-// Dynamic LDS beyond 64 KiB has to be asked for once per kernel.
+// Dynamic LDS beyond 64 KiB has to be asked for.  The limit belongs to the
+// kernel, which all plans and threads of the process share: every launch asks
+// for the same most that any shape takes, so that none lowers it between
+// another's asking and its launch.
 template <typename F>
 static int allow_lds(F *kernel, size_t bytes) {
   if (bytes <= 64 * 1024) return FLUTAS_OK;
   FL_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
-                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kGenLds));
   return FLUTAS_OK;
 }
 

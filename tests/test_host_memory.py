@@ -48,3 +48,24 @@ p.destroy(); f.free(); g.free(); d32.free()
 api.lib.flutas_fft_cleanup()
 assert sim.sim_used() == 0, "device memory left"
 """, tmp_path)
+
+
+def test_plans_do_not_lower_each_others_lds_limit(tmp_path):
+    """The dynamic LDS limit of a kernel is one for the process: plans and
+    transforms of other lengths must not lower it between another thread's
+    setting and its launch."""
+    hipsim.run("""
+big = [(1998, 1000, 20), (1400, 706, 20), (1362, 1362, 20), (1026, 2046, 20)]
+fields = [(plan(ng, **kw), field(ng), field(ng)) for ng in big
+          for kw in ({}, dict(precision=32))]
+d = api.DeviceArray((2046, 40))
+for _ in range(2):
+    for p, f, g in fields:
+        api.lib.flutas_psolve_solve_into(C.c_void_p(p._h), f.c, g.c)
+    for n in (2046, 1400, 1026):
+        api.fft_lines("R2HC", d, n, 20)
+lds = {l[3] for l in launches()}
+assert len([v for v in lds if v > 64 * 1024]) >= 3, lds
+assert sim.sim_count(2) == 0
+assert sim.sim_lowered() == 0
+""", tmp_path)
