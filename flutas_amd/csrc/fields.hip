@@ -1178,11 +1178,13 @@ __global__ void __launch_bounds__(256) k_halo(HaloArgs<T> a) {
 }
 
 // The stages (at most one per direction and position with a rule) on nf fields
-// as one launch: every n above 2 nh and within the kernel's 32-bit counts.
+// as one launch: every n above 2 nh and within the kernel's 32-bit counts, the
+// threads of all faces together fewer than the 2^32 that a launch holds.
 static bool halo_one(const int n[3], int nh) {
   for (int d = 0; d < 3; ++d)
     if (n[d] <= 2 * nh || n[d] + 2 * nh > 65535) return false;
-  return true;
+  const double x = n[0], y = n[1], z = n[2], np = 2 * nh + 1;
+  return y * z + np * x * (y + z) + np * np * (x + y + z + 2 * nh) + 256 * (2 * np + 2) < 4294967296.0;
 }
 template <typename T>
 static int launch_halo(const FaceArgs<T> *st, int nst, T *const *fld, int nf, const int n[3],

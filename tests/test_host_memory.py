@@ -69,3 +69,23 @@ assert len([v for v in lds if v > 64 * 1024]) >= 3, lds
 assert sim.sim_count(2) == 0
 assert sim.sim_lowered() == 0
 """, tmp_path)
+
+
+@pytest.mark.parametrize("ng", [(40000, 40000, 4), (4, 40000, 40000), (40000, 4, 40000),
+                                (33000, 33000, 4)])
+def test_boundary_calls_on_large_flat_grids(tmp_path, ng):
+    """A launch holds fewer than 2^32 threads; faces beyond that go one by one."""
+    hipsim.run(f"""
+ng = {ng}
+# 60 GB of addresses, no memory: nothing here touches the fields
+p = api.DeviceArray([1])
+fake = type("F", (api.DeviceArray,), dict(__init__=lambda s: None, free=lambda s: None))
+a = fake()
+a.shape, a.dtype, a.ptr = tuple(n + 2 for n in ng), np.dtype(np.float64), p.ptr
+dz = np.full(ng[2] + 2, 0.5)
+for cbc in ("PPPPPP", "DDNNND", "PPPPNN"):
+    api.boundp(cbc, ng, (0.0,) * 6, (1.0, 1.0, 1.0), 0.5, 0.5, a)
+    api.boundp_halo(cbc, ng, (0.0,) * 6, 1, 1, (1.0, 1.0, 1.0), dz, dz, a)
+api.bounduvw("D" * 18, ng, np.zeros(18), 1, 1, [0] * 6, (1.0, 1.0, 1.0), dz, dz, a, a, a)
+assert sim.sim_count(2) == 0 and len(launches()) > 0
+""", tmp_path)
