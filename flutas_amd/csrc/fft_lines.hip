@@ -530,9 +530,10 @@ void LineTables::release() {
 // Tables of the stand-alone transforms, kept between calls as the plan of a
 // program that transforms the same lengths again (the reference makes its
 // FFTW plans once): tables built in each call cost it 340 us beside 70 us of
-// kernel (256 points).  The kTableLengths lengths used last stay, at most 1.1 MB
-// each; a caller holds its tables until its stream is done with them, so one
-// thread's eviction never takes another's.  clear_line_tables() gives them back.
+// kernel (256 points).  The kTableLengths lengths used last stay, at most 0.7 MB
+// each (8192 points, the longest lines that a kernel takes); a caller holds its
+// tables until its stream is done with them, so one thread's eviction never
+// takes another's.  clear_line_tables() gives them back.
 namespace {
 constexpr size_t kTableLengths = 16;
 struct KeptTables {
@@ -599,7 +600,7 @@ int launch_lines(const LineTables &tab, int kind, const Tin *in, Tout *out,
   if (m != tab.n) return fail(FLUTAS_EINVAL, "line length does not match plan");
   // lines per block: as many as fit 64 KiB of LDS (two buffers), <= 16
   const size_t per_line = 2 * (size_t)m * sizeof(T);
-  int lpb = (int)std::min<size_t>(16, (64 * 1024) / per_line);
+  int lpb = (int)std::min<size_t>(16, kLineLds / per_line);
   if (lpb < 1) return fail(FLUTAS_EUNSUPPORTED, "line too long for one workgroup");
   lpb = std::min(lpb, g.L1);
   dim3 grid((g.L1 + lpb - 1) / lpb, g.L2);

@@ -130,6 +130,9 @@ struct LineGeom {
   long long os1, os2, ose;
 };
 
+// LDS of one workgroup of launch_lines, which holds two buffers of each of its
+// lines: the longest line it takes fills it.
+constexpr size_t kLineLds = 64 * 1024;
 // Launch one batched line transform: in -> out (may alias only if the
 // geometries are identical).  Tin/Tout storage, T arithmetic.
 template <typename T, typename Tin, typename Tout>

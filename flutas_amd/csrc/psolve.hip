@@ -1140,6 +1140,9 @@ static int fft_guru_impl(int kind, int n, long long stride, int howmany1, long l
   // other kinds an even n
   if (kind != K_REDFT00 && kind != K_RODFT00 && (n & 1))
     return fail(FLUTAS_EINVAL, "line length must be even for this kind");
+  // no kernel runs these: refused before any table is made and kept
+  if ((size_t)n > kLineLds || 2 * sizeof(T) * dft_length(kind, n) > kLineLds)
+    return fail(FLUTAS_EUNSUPPORTED, "line too long for one workgroup");
   std::shared_ptr<const LineTables> tab;
   FL_TRY(line_tables(dft_length(kind, n), &tab));
   LineGeom g;

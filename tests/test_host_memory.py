@@ -89,3 +89,34 @@ for cbc in ("PPPPPP", "DDNNND", "PPPPNN"):
 api.bounduvw("D" * 18, ng, np.zeros(18), 1, 1, [0] * 6, (1.0, 1.0, 1.0), dz, dz, a, a, a)
 assert sim.sim_count(2) == 0 and len(launches()) > 0
 """, tmp_path)
+
+
+def test_refused_transforms_keep_no_tables(tmp_path):
+    """Lines too long for a workgroup's LDS (64 KB, two buffers) are refused
+    without tables; the longest that run keep no more than is stated, and
+    flutas_fft_cleanup gives all of it back."""
+    hipsim.run("""
+def lines(n, f32=False, kind="REDFT10"):
+    fn = api.lib.flutas_fft_guru_f32 if f32 else api.lib.flutas_fft_guru
+    ct = C.c_float if f32 else C.c_double
+    code = dict(REDFT10=5, REDFT00=3, RODFT00=7)[kind]
+    return fn(C.c_int(code), C.c_int(n), C.c_longlong(1), C.c_int(1), C.c_longlong(n), C.c_int(1),
+              C.c_longlong(0), C.cast(C.c_void_p(d.ptr), C.POINTER(ct)))
+
+d = api.DeviceArray([1 << 14])
+before = sim.sim_used()
+for n in (4098, 1 << 16, 1 << 20, (1 << 31) - 2):
+    assert lines(n) == api.FLUTAS_EUNSUPPORTED
+    assert lines(n, kind="REDFT00") == api.FLUTAS_EUNSUPPORTED
+    assert lines(n + 1 if n < 1 << 30 else n, kind="RODFT00") == api.FLUTAS_EUNSUPPORTED
+assert lines(8194, True) == api.FLUTAS_EUNSUPPORTED
+assert lines(2050, kind="REDFT00") == api.FLUTAS_EUNSUPPORTED
+assert sim.sim_used() == before and not launches()
+assert lines(4096) == 0 and lines(8192, True) == 0 and lines(2049, kind="REDFT00") == 0
+assert 0 < sim.sim_used() - before <= 2 * 700000
+for n in range(8192, 8192 - 400, -2):
+    lines(n, True)
+assert sim.sim_used() - before <= 16 * 700000
+assert api.lib.flutas_fft_cleanup() == 0
+assert sim.sim_used() == before
+""", tmp_path)
