@@ -656,7 +656,15 @@ int solve_refined(flutas_psolve *h, const double *fsrc, double *p, hipStream_t s
     FL_TRY(reduce_max(h, np, s, &rmax, n1, &fmax));
     if (n1 > 0) {
       n1 = 0;
-      if (!(fmax == fmax) || std::isinf(fmax)) return fail(FLUTAS_ENONFINITE, "right-hand side holds NaN or Inf");
+      if (!(fmax == fmax) || std::isinf(fmax)) {
+        // in place at lengths without a compiled plan the caller gets its
+        // right-hand side back
+        if (fsrc == p && !h->compiled()) {
+          FL_HIP(hipMemcpyAsync(p, h->F, sizeof(double) * nhalo, hipMemcpyDeviceToDevice, s));
+          FL_HIP(hipStreamSynchronize(s));
+        }
+        return fail(FLUTAS_ENONFINITE, "right-hand side holds NaN or Inf");
+      }
     }
     rel = (fmax > 0.0) ? rmax / fmax : rmax;
     if (!(rel == rel)) return fail(FLUTAS_ENONFINITE, "residual is NaN");

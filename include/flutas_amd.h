@@ -101,7 +101,8 @@ int flutas_psolve_rhsb_device(const flutas_psolve *h, const double **rhsbx,
  * the Poisson equation in place on the interior of the device array p
  * (0:nx+1,0:ny+1,0:nz+1); halo values are neither read nor written.
  * Returns when the result is in p.  A right-hand side holding NaN or Inf
- * returns FLUTAS_ENONFINITE (p then holds non-finite values). */
+ * returns FLUTAS_ENONFINITE (p then holds non-finite values; refined plans
+ * with a line length that has no compiled plan leave it as it came). */
 int flutas_psolve_solve(flutas_psolve *h, double *p);
 
 /* Same, enqueued on the library stream; returns immediately.  The refined

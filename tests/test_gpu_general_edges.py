@@ -32,3 +32,22 @@ def test_f32_nonfinite_is_reported(api, oracle, ng, bad):
         assert _solve32(api, plan, d) == code
         assert np.all(np.isfinite(d.to_host())) == (code == 0)
     plan.destroy()
+
+
+@pytest.mark.parametrize("bad", [np.nan, -np.inf])
+@pytest.mark.parametrize("ng", [(36, 64, 20), (64, 300, 20), (90, 154, 20)])
+def test_refined_nonfinite_gives_the_right_hand_side_back(api, oracle, ng, bad):
+    """In place the field comes back bit for bit, halo included; out of place
+    the right-hand side is not written."""
+    _, _, dzci, dzfi, _, _ = z_metrics(oracle, ng[2], 0.0, 1.0)
+    plan = api.PoissonPlan(ng, tuple(float(n) for n in ng), dzci, dzfi, "PPDDNN",
+                           precision=api.FP32_REFINE, tol=1e-8)
+    f = np.asfortranarray(np.random.default_rng(2).standard_normal([n + 2 for n in ng]))
+    f[5, 7, 4] = bad
+    d, p = api.DeviceArray.from_host(f), api.DeviceArray(f.shape)
+    for call in (lambda: plan.solve(d), lambda: plan.solve_async(d), lambda: plan.solve_into(d, p)):
+        with pytest.raises(api.FlutasError) as e:
+            call()
+        assert e.value.code == api.FLUTAS_ENONFINITE
+        np.testing.assert_array_equal(d.to_host(), f)
+    plan.destroy()
