@@ -73,7 +73,7 @@ __global__ void __launch_bounds__(256)
     if (k % gp == 0) {
       const long long o = ((long long)i * ngrp + k / gp) * ny + j;
       ckd[o] = dp;
-      ckm[o] = mp;
+      if (nchunk > 1) ckm[o] = mp;
       if (per) ckq[o] = qp;
     }
     if (k < msys) {
@@ -183,8 +183,9 @@ int fused_slab_residency(int ny, int elem_bytes, int periodic, int *r2, int *r3)
 }
 
 size_t zchunk_doubles(int nx, int ny, int ngrp, int nchunk, bool per) {
-  const size_t col = (size_t)nx * ny;
-  return col * (3 * (size_t)ngrp + (size_t)nchunk * zc_tab_slots(per) + 1 +
+  // values at a plane group: d, with two chunks or more m, with periodic z q2
+  const size_t col = (size_t)nx * ny, grp = 1 + (nchunk > 1) + per;
+  return col * (grp * ngrp + (size_t)nchunk * zc_tab_slots(per) + per +
                 (size_t)nchunk * zc_side_slots(per));
 }
 
@@ -197,10 +198,14 @@ int build_zchunk_tables(double *mem, ZChunks *zc, int nx, int ny, int nz, int ms
     return fail(FLUTAS_EINVAL, "z chunks: bad chunk shape");
   const int ngrp = (nz + gp - 1) / gp;
   const size_t col = (size_t)nx * ny;
-  double *ckd = mem, *ckm = ckd + col * ngrp, *ckq = ckm + col * ngrp;
-  double *tab = ckq + col * ngrp;
+  // One chunk carries nothing in, its multipliers meet a zero: it reads d in
+  // their place (the same lines again, no bytes of its own).
+  double *ckd = mem, *ckm = nchunk > 1 ? ckd + col * ngrp : ckd;
+  double *ckq = ckm + col * ngrp;
+  double *tab = per ? ckq + col * ngrp : ckq;
   double *den = tab + col * nchunk * zc_tab_slots(per);
-  double *side = den + col;
+  double *side = per ? den + col : den;
+  if (!per) ckq = den = nullptr;
   const int threads = 256;
   const long long blocks = ((long long)col + threads - 1) / threads;
   if (elem_bytes == 8)

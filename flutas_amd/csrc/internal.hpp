@@ -218,7 +218,7 @@ struct ZChunks {
 __host__ __device__ constexpr int zc_tab_slots(bool per) { return per ? 4 : 3; }
 __host__ __device__ constexpr int zc_side_slots(bool per) { return per ? 3 : 2; }
 // Tables of a plan's chunking (one thread per column; mem holds
-// 3 ngrp + nchunk tab slots + 1 + nchunk side slots values per column).
+// zchunk_doubles values).
 size_t zchunk_doubles(int nx, int ny, int ngrp, int nchunk, bool per);
 int build_zchunk_tables(double *mem, ZChunks *zc, int nx, int ny, int nz, int msys, int gp,
                         int cpl, int nchunk, bool per, int pin, int elem_bytes,

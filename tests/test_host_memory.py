@@ -120,3 +120,28 @@ assert sim.sim_used() - before <= 16 * 700000
 assert api.lib.flutas_fft_cleanup() == 0
 assert sim.sim_used() == before
 """, tmp_path)
+
+
+@pytest.mark.parametrize("ng,gp", [((60, 300, 128), 8), ((6, 1200, 64), 4), ((66, 154, 128), 16)])
+@pytest.mark.parametrize("z", ["NN", "PP"])
+def test_chunk_tables_hold_what_is_read(tmp_path, ng, gp, z):
+    """Per column and plane group d, with two chunks or more m, with periodic z
+    q2; beyond that a few values per column and chunk."""
+    hipsim.run(f"""
+nx, ny, nz = {ng}
+per = {z == "PP"}
+p = plan({ng}, "PPDD{z}")
+
+def used(n):
+    assert p.set_zchunks(n) == n
+    return sim.sim_used()
+
+def tables(n):
+    slots = n * (7 if per else 5) + per
+    return 8 * nx * ny * ((1 + (n > 1) + per) * -(-nz // {gp}) + slots)
+
+assert used(4) - used(1) == tables(4) - tables(1)
+total = used(1)
+field8 = 8 * nx * ny * nz
+assert total - tables(1) < 1.3 * field8 + 4e6, (total, tables(1), field8)
+""", tmp_path)
