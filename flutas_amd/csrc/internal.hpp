@@ -187,8 +187,8 @@ __host__ __device__ inline WStride plane_major(int nx, int pitch) {
 // of 8 are 1-2% slower, so those stay plane-major.  The FP32 chain of the
 // refined mode is 2% faster plane-major, and the batched solves measure the
 // same either way (they stay plane-major).
-__host__ __device__ inline WStride fused_layout_fp64(int nx, int ny, int nz) {
-  if (ny != 512) return plane_major(nx, line_pitch(ny, 8));
+__host__ __device__ inline WStride fused_layout_fp64(int nx, int ny, int nz, int pitch) {
+  if (ny != 512) return plane_major(nx, pitch);
   int lb = 0;
   while (lb < 3 && ((nx >> lb) & 1) == 0) ++lb;
   return slab_blocked(ny, nz, lb);

@@ -162,6 +162,7 @@ struct flutas_psolve {
   double *d_rhsbx = nullptr, *d_rhsby = nullptr, *d_rhsbz = nullptr;
   double *W64 = nullptr;   // spectral work field (FP64 mode)
   float *W32 = nullptr;    // spectral work field (refined mode)
+  int pitch64 = 0, pitch32 = 0;  // distance of their y-lines
   double *TK = nullptr;    // z elimination checkpoints of the line path
   double *F = nullptr;     // copy of the right-hand side (refined mode)
   float *R32 = nullptr;    // residual (refined mode)
@@ -196,9 +197,18 @@ struct flutas_psolve {
 
 namespace {
 
-// Values of a work field (see line_pitch).
-size_t work_values(const flutas_psolve *h, int elem_bytes) {
-  return (size_t)h->nx * line_pitch(h->ny, elem_bytes) * h->nz;
+// A work field: y-lines at line_pitch, or dense where that does not fit (or the
+// plan is a lean one).
+template <typename T>
+hipError_t alloc_work(flutas_psolve *h, T **W, int *pitch, bool lean) {
+  hipError_t e = hipErrorOutOfMemory;
+  for (const int q : {line_pitch(h->ny, sizeof(T)), h->ny}) {
+    if (e == hipSuccess || (lean && q != h->ny)) continue;
+    (void)hipGetLastError();
+    e = hipMalloc((void **)W, (size_t)h->nx * q * h->nz * sizeof(T));
+    *pitch = q;
+  }
+  return e;
 }
 
 template <typename T>
@@ -210,13 +220,16 @@ int dev_upload(T **d, const std::vector<T> &h) {
 }
 
 void release(flutas_psolve *h) {
-  for (void *p : {(void *)h->d_lamx, (void *)h->d_lamy, (void *)h->d_a,
-                  (void *)h->d_b, (void *)h->d_c, (void *)h->d_rhsbx,
-                  (void *)h->d_rhsby, (void *)h->d_rhsbz, (void *)h->W64,
-                  (void *)h->W32, (void *)h->TK, (void *)h->F,
-                  (void *)h->R32, (void *)h->part, (void *)h->CK, (void *)h->zcs.mem,
-                  (void *)h->zcs32.mem})
-    if (p) (void)hipFree(p);
+  for (void **p : {(void **)&h->d_lamx, (void **)&h->d_lamy, (void **)&h->d_a,
+                   (void **)&h->d_b, (void **)&h->d_c, (void **)&h->d_rhsbx,
+                   (void **)&h->d_rhsby, (void **)&h->d_rhsbz, (void **)&h->W64,
+                   (void **)&h->W32, (void **)&h->TK, (void **)&h->F,
+                   (void **)&h->R32, (void **)&h->part, (void **)&h->CK, (void **)&h->zcs.mem,
+                   (void **)&h->zcs32.mem}) {
+    if (*p) (void)hipFree(*p);
+    *p = nullptr;
+  }
+  h->zcs = h->zcs32 = ChunkSet{};
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   h->ev.clear();
   if (h->nf_host) (void)hipHostFree(h->nf_host);
@@ -506,8 +519,8 @@ int spectral(flutas_psolve *h, const Tin *in, bool in_halo, Tout *out,
     // the singular column takes p(last) = 0 for NN and for periodic z
     const int per = (h->cbc[4] == 'P');
     const int pin = (h->cbc[4] == 'N' && h->cbc[5] == 'N') || per;
-    const WStride ws = sizeof(T) == 8 ? fused_layout_fp64(nx, ny, nz)
-                                      : plane_major(nx, line_pitch(ny, 4));
+    const WStride ws = sizeof(T) == 8 ? fused_layout_fp64(nx, ny, nz, h->pitch64)
+                                      : plane_major(nx, h->pitch32);
     if (h->gx)
       FL_TRY((launch_gen_x_fwd<T, Tin>(h->tx, h->kinds[0], in, is1, is2, W, ws, ny, nz,
                                        absmax_part, nf_flag, h->seq, s)));
@@ -572,9 +585,7 @@ int solve_fp64(flutas_psolve *h, const double *f, double *p, hipStream_t s) {
 // solve in FP32.  The FP32 work field and the chunk tables are made on
 // first use when the plan is an FP64 one.
 int solve_f32(flutas_psolve *h, const float *f, float *p, hipStream_t s) {
-  if (!h->W32) {
-    FL_HIP(hipMalloc((void **)&h->W32, work_values(h, 4) * sizeof(float)));
-  }
+  if (!h->W32) FL_HIP(alloc_work(h, &h->W32, &h->pitch32, !h->fused));
   if (!h->has32 && h->fused && !h->gy && h->precision == FLUTAS_FP64) {
     h->has32 = true;
     build_chunks32(h);
@@ -685,6 +696,75 @@ int solve_refined(flutas_psolve *h, const double *fsrc, double *p, hipStream_t s
   h->last_iters = it;
   h->last_relres = rel;
   return FLUTAS_OK;
+}
+
+// Tables and device memory of a plan whose host side is set.  lean: work fields
+// without padding between lines, lengths without a compiled plan on the line
+// path, which needs no chunk tables.
+int setup_device(flutas_psolve *h, bool lean) {
+  const size_t N = (size_t)h->nx * h->ny * h->nz;
+  const size_t nhalo = (size_t)(h->nx + 2) * (h->ny + 2) * (h->nz + 2);
+  const bool fp64 = h->precision == FLUTAS_FP64, per = h->cbc[4] == 'P';
+  // the fused pipeline covers the compiled line lengths, and the general
+  // kernels every other even length up to 2048
+  // (the tile transforms cover the R2HC, DCT-II/III, DCT-IV and DST kinds
+  // run forward in P1/P2 and backward in P3/P4)
+  const char *env = std::getenv("FLUTAS_UNFUSED");
+  const bool tile_kinds = fused_forward_kind(h->kinds[0]) && fused_forward_kind(h->kinds[2]);
+  const bool gx = !fused_supported(h->nx), gy = !fused_supported(h->ny);
+  h->fused = (!gx || (general_supported(h->nx) && !lean)) &&
+             (!gy || (general_supported(h->ny) && !lean)) && h->nz >= 3 && tile_kinds &&
+             !(env && env[0] == '1');
+  h->gx = h->fused && gx;
+  h->gy = h->fused && gy;
+  // (a direction on the general kernels needs their tables only)
+  FL_TRY(h->gx ? build_general_tables(h->tx, h->nx) : h->tx.build(h->nx));
+  FL_TRY(h->gy ? build_general_tables(h->ty, h->ny) : h->ty.build(h->ny));
+  if (!gx) FL_TRY(build_fused_twiddles(h->tx));
+  if (!gy) FL_TRY(build_fused_twiddles(h->ty));
+  FL_TRY(dev_upload(&h->d_lamx, h->lamx));
+  FL_TRY(dev_upload(&h->d_lamy, h->lamy));
+  FL_TRY(dev_upload(&h->d_a, h->a));
+  FL_TRY(dev_upload(&h->d_b, h->b));
+  FL_TRY(dev_upload(&h->d_c, h->c));
+  FL_TRY(dev_upload(&h->d_rhsbx, h->rhsbx));
+  FL_TRY(dev_upload(&h->d_rhsby, h->rhsby));
+  FL_TRY(dev_upload(&h->d_rhsbz, h->rhsbz));
+  hipError_t e = hipSuccess;
+  if (fp64) {
+    e = alloc_work(h, &h->W64, &h->pitch64, lean || !h->fused);
+  } else {
+    e = alloc_work(h, &h->W32, &h->pitch32, lean || !h->fused);
+    if (e == hipSuccess) e = hipMalloc((void **)&h->R32, N * sizeof(float));
+    if (e == hipSuccess) e = hipMalloc((void **)&h->F, nhalo * sizeof(double));
+  }
+  if (h->fused && !h->gy) {
+    const int gp = fused_group_planes(h->ny, plan_elem(h));
+    // one checkpoint per plane group (two values per column for periodic z)
+    const size_t ngrp = (h->nz + gp - 1) / gp;
+    const size_t nck = std::max<size_t>(1, ngrp) * (per ? 2 : 1);
+    if (e == hipSuccess) e = hipMalloc((void **)&h->CK, (size_t)h->nx * nck * h->ny * sizeof(double));
+  } else if (!h->fused) {
+    const size_t ntk = thomas_checkpoint_doubles(h->nx, h->ny, h->nz, per);
+    if (e == hipSuccess) e = hipMalloc((void **)&h->TK, ntk * sizeof(double));
+  }
+  if (e == hipSuccess) e = hipHostMalloc((void **)&h->nf_host, 4 * sizeof(double), hipHostMallocDefault);
+  if (e == hipSuccess) {
+    *h->nf_host = 0;
+    e = hipHostGetDevicePointer((void **)&h->nf_dev, h->nf_host, 0);
+  }
+  h->nres = residual_blocks(h->nx, h->ny, h->nz);
+  h->nx1 = !h->fused || fp64 ? 0
+           : (size_t)(h->gx ? gen_x_fwd_blocks(h->nx, 4, h->ny, h->nz)
+                            : x_fwd_blocks(h->tx, 4, h->ny, h->nz));
+  if (e == hipSuccess) e = hipMalloc((void **)&h->part, (h->nres + h->nx1) * sizeof(double));
+  if (e != hipSuccess)
+    return fail(FLUTAS_ENOMEM, std::string("device allocation: ") + hipGetErrorString(e));
+  const char *zenv = std::getenv("FLUTAS_ZCHUNKS");
+  h->zreq = zenv ? std::atoi(zenv) : 0;
+  const int rc = set_zchunks(h, zenv ? h->zreq : default_zchunks(h, plan_elem(h)));
+  // without tables compiled y lines walk whole slabs
+  return rc && !zenv && h->fused && !h->gy ? FLUTAS_OK : rc;
 }
 
 }  // namespace
@@ -808,67 +888,14 @@ int flutas_psolve_create(const int ng[3], const char cbc[6], const double bc[6],
     const double dlf[2] = {1.0 / zfi[1], 1.0 / zfi[h->nz]};
     bc_rhs(cbc + 4, bc + 4, dlc, dlf, c_or_f[2], (long)h->nx * h->ny, h->rhsbz);
   }
-  int rc = FLUTAS_OK;
-  const size_t N = (size_t)h->nx * h->ny * h->nz;
-  const size_t nhalo = (size_t)(h->nx + 2) * (h->ny + 2) * (h->nz + 2);
-  do {
-    // the fused pipeline covers the compiled line lengths, and the general
-    // kernels every other even length up to 2048
-    // (the tile transforms cover the R2HC, DCT-II/III, DCT-IV and DST kinds
-    // run forward in P1/P2 and backward in P3/P4)
-    const char *env = std::getenv("FLUTAS_UNFUSED");
-    const bool tile_kinds = fused_forward_kind(h->kinds[0]) && fused_forward_kind(h->kinds[2]);
-    const bool gx = !fused_supported(h->nx), gy = !fused_supported(h->ny);
-    h->fused = (!gx || general_supported(h->nx)) && (!gy || general_supported(h->ny)) &&
-               h->nz >= 3 && tile_kinds && !(env && env[0] == '1');
-    h->gx = h->fused && gx;
-    h->gy = h->fused && gy;
-    // (a direction on the general kernels needs their tables only)
-    if ((rc = h->gx ? build_general_tables(h->tx, h->nx) : h->tx.build(h->nx))) break;
-    if ((rc = h->gy ? build_general_tables(h->ty, h->ny) : h->ty.build(h->ny))) break;
-    if (!gx && (rc = build_fused_twiddles(h->tx))) break;
-    if (!gy && (rc = build_fused_twiddles(h->ty))) break;
-    if ((rc = dev_upload(&h->d_lamx, h->lamx))) break;
-    if ((rc = dev_upload(&h->d_lamy, h->lamy))) break;
-    if ((rc = dev_upload(&h->d_a, h->a))) break;
-    if ((rc = dev_upload(&h->d_b, h->b))) break;
-    if ((rc = dev_upload(&h->d_c, h->c))) break;
-    if ((rc = dev_upload(&h->d_rhsbx, h->rhsbx))) break;
-    if ((rc = dev_upload(&h->d_rhsby, h->rhsby))) break;
-    if ((rc = dev_upload(&h->d_rhsbz, h->rhsbz))) break;
-    hipError_t e = hipSuccess;
-    if (precision == FLUTAS_FP64) {
-      e = hipMalloc((void **)&h->W64, work_values(h, 8) * sizeof(double));
-    } else {
-      e = hipMalloc((void **)&h->W32, work_values(h, 4) * sizeof(float));
-      if (e == hipSuccess) e = hipMalloc((void **)&h->R32, N * sizeof(float));
-      if (e == hipSuccess) e = hipMalloc((void **)&h->F, nhalo * sizeof(double));
-    }
-    if (h->fused && !h->gy) {
-      const int gp = fused_group_planes(h->ny, precision == FLUTAS_FP64 ? 8 : 4);
-      // one checkpoint per plane group (two values per column for periodic z)
-      const size_t ngrp = (h->nz + gp - 1) / gp;
-      const size_t nck = std::max<size_t>(1, ngrp) * (cbc[4] == 'P' ? 2 : 1);
-      if (e == hipSuccess) e = hipMalloc((void **)&h->CK, (size_t)h->nx * nck * h->ny * sizeof(double));
-    } else if (!h->fused) {
-      const size_t ntk = thomas_checkpoint_doubles(h->nx, h->ny, h->nz, cbc[4] == 'P');
-      if (e == hipSuccess) e = hipMalloc((void **)&h->TK, ntk * sizeof(double));
-    }
-    if (e == hipSuccess) e = hipHostMalloc((void **)&h->nf_host, 4 * sizeof(double), hipHostMallocDefault);
-    if (e == hipSuccess) {
-      *h->nf_host = 0;
-      e = hipHostGetDevicePointer((void **)&h->nf_dev, h->nf_host, 0);
-    }
-    h->nres = residual_blocks(h->nx, h->ny, h->nz);
-    h->nx1 = (h->fused && precision == FLUTAS_FP32_REFINE) ? (size_t)(h->gx ? gen_x_fwd_blocks(h->nx, 4, h->ny, h->nz)
-                                           : x_fwd_blocks(h->tx, 4, h->ny, h->nz))
-                          : 0;
-    if (e == hipSuccess) e = hipMalloc((void **)&h->part, (h->nres + h->nx1) * sizeof(double));
-    if (e != hipSuccess) { rc = fail(FLUTAS_ENOMEM, std::string("device allocation: ") + hipGetErrorString(e)); break; }
-    const char *zenv = std::getenv("FLUTAS_ZCHUNKS");
-    h->zreq = zenv ? std::atoi(zenv) : 0;
-    if ((rc = set_zchunks(h, zenv ? h->zreq : default_zchunks(h, plan_elem(h))))) break;
-  } while (0);
+  // Padded work fields and chunk tables take memory that a plan can do without:
+  // where they do not fit it is a lean one.
+  int rc = setup_device(h, false);
+  if (rc && (h->gx || h->gy || line_pitch(h->ny, plan_elem(h)) != h->ny)) {
+    release(h);
+    (void)hipGetLastError();
+    rc = setup_device(h, true);
+  }
   if (rc) {
     release(h);
     delete h;
@@ -1091,7 +1118,7 @@ int flutas_psolve_time_stage(flutas_psolve *h, const double *f, double *p, int s
   const int nx = h->nx, ny = h->ny, nz = h->nz;
   const int per = (h->cbc[4] == 'P');
   const int pin = (h->cbc[4] == 'N' && h->cbc[5] == 'N') || per;
-  const WStride ws = fused_layout_fp64(nx, ny, nz);
+  const WStride ws = fused_layout_fp64(nx, ny, nz, h->pitch64);
   hipEvent_t e0, e1;
   FL_HIP(hipEventCreate(&e0));
   FL_HIP(hipEventCreate(&e1));

@@ -55,6 +55,7 @@ static int kernel_of(const void *f) {
 }
 
 /* ---- memory ---- */
+static __thread hipError_t last;  /* what hipGetLastError returns */
 hipError_t hipMalloc(void **p, size_t n) {
   hipError_t e = hipErrorOutOfMemory;
   *p = NULL;
@@ -75,6 +76,7 @@ hipError_t hipMalloc(void **p, size_t n) {
     }
   }
   pthread_mutex_unlock(&mu);
+  if (e != hipSuccess) last = e;
   return e;
 }
 hipError_t hipFree(void *p) {
@@ -121,7 +123,6 @@ hipError_t hipGetLastError(void);
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "hipsim error"; }
 
 /* ---- kernels ---- */
-static __thread hipError_t last;
 hipError_t hipGetLastError(void) { hipError_t e = last; last = hipSuccess; return e; }
 static __thread struct { dim3 g, b; size_t lds; hipStream_t s; } call;
 hipError_t __hipPushCallConfiguration(dim3 g, dim3 b, size_t lds, hipStream_t s) {

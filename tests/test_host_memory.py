@@ -145,3 +145,53 @@ total = used(1)
 field8 = 8 * nx * ny * nz
 assert total - tables(1) < 1.3 * field8 + 4e6, (total, tables(1), field8)
 """, tmp_path)
+
+
+@pytest.mark.parametrize("ng,cbc,kw", [
+    ((360, 300, 64), "PPDDNN", "{}"), ((6, 1200, 100), "PPDDPP", "{}"),
+    ((128, 154, 90), "NNDDNN", "dict(precision=32)"), ((300, 64, 90), "PPDDPP", "{}"),
+    ((100, 100, 100), "PPDDNN", "{}"), ((128, 200, 100), "PPDDPP", "dict(precision=32)")])
+def test_plans_fit_where_the_line_path_fits(tmp_path, ng, cbc, kw):
+    """A plan needs no more memory than its work field, the elimination's
+    checkpoints and the small tables: the padding and the chunk tables are
+    left out where they do not fit, and the plan solves all the same."""
+    hipsim.run(f"""
+import os
+ng, cbc = {ng}, "{cbc}"
+compiled = all(n in (64, 100, 128, 200) for n in ng[:2])
+nx, ny, nz = ng
+def make():
+    before = sim.sim_used()
+    p = plan(ng, cbc, **{kw})
+    return p, sim.sim_used() - before
+if compiled:
+    # no line path to compare with: a dense field, one value per 8 planes and column
+    # (two for periodic z), and what is small
+    fp64, groups = not {kw}, -(-nz // 8)
+    need = 8 * nx * ny * (nz + groups * (2 if cbc[4] == "P" else 1))
+    need += 0 if fp64 else 8 * (nx + 2) * (ny + 2) * (nz + 2)
+    need += 16 * (nx * ny + nx * nz + ny * nz) + 400000
+else:
+    os.environ["FLUTAS_UNFUSED"] = "1"
+    p, need = make()
+    p.destroy()
+    del os.environ["FLUTAS_UNFUSED"]
+f, g = field(ng), field(ng)
+rich, most = make()
+rich.destroy()
+sim.sim_limit(sim.sim_used() + need)
+p, got = make()
+assert got <= need < most, (got, need, most)
+sim.sim_reset()
+assert api.lib.flutas_psolve_solve_into(C.c_void_p(p._h), f.c, g.c) in (0, api.FLUTAS_ENOTCONV)
+assert sim.sim_count(2) == 0 and len(launches()) >= 4
+p.destroy()
+# an FP32 field on an FP64 plan: the work field dense, whole slabs
+sim.sim_limit(UNLIMITED)
+if not {kw}:
+    d32 = field(ng, np.float32)
+    p, got = make()
+    sim.sim_limit(sim.sim_used() + 4 * nx * ny * nz)
+    assert solve32(p, d32) == 0 and sim.sim_count(2) == 0
+    p.destroy()
+""", tmp_path)
