@@ -3,6 +3,8 @@
 #include "fused_chunk.hpp"
 #include "fused_host.hpp"
 
+#include <type_traits>
+
 namespace flutas {
 
 template <typename T, int NC, int GP, int NT, bool PER>
@@ -45,12 +47,17 @@ __global__ void __launch_bounds__(NT, slab_waves_per_simd(NT))
 // the second solution p2 at every chunk start and the closing row's
 // denominator (b(m) + lam) + c(m) p2(0) + a(m) p2(m-1).
 // The pivot reciprocals are those of the chain the tables serve (zrcp<T>).
+// Bound by the chain of a column's pivots, one thread's whole work: the rows
+// of a group without one of the first, last and closing rows run straight
+// through, up to eight at a time with their coefficients loaded ahead (a new plan
+// of 32x32x2048 periodic z 1.81 -> 0.84 ms, 2x2x1000 0.78 -> 0.37).
+// GP: planes of a group, 0 for gp.
 constexpr int kZcMaxGroup = 16;
-template <typename T>
+template <typename T, bool PER, int GP>
 __global__ void __launch_bounds__(256)
     k_zchunk_tables(double *__restrict__ ckd, double *__restrict__ ckm, double *__restrict__ ckq,
                     double *__restrict__ tab, double *__restrict__ den, int nx, int ny, int nz,
-                    int msys, int gp, int cpl, int nchunk, int per, int pin,
+                    int msys, int gp_, int cpl, int nchunk, int pin,
                     const double *__restrict__ lamx, const double *__restrict__ lamy,
                     const double *__restrict__ a, const double *__restrict__ b,
                     const double *__restrict__ c) {
@@ -59,25 +66,59 @@ __global__ void __launch_bounds__(256)
   if (col >= (long long)nx * ny) return;
   const int i = (int)(col / ny), j = (int)(col - (long long)i * ny);
   const double lam = lamx[i] + lamy[j];
+  const int gp = GP ? GP : gp_;
   const int ngrp = (nz + gp - 1) / gp;
-  const int TS = zc_tab_slots(per != 0);
+  constexpr int TS = zc_tab_slots(PER), H = GP == 0 ? 1 : (GP < 8 ? GP : 8);
   double dp = 0.0, mp = 1.0, qp = 0.0, w = 1.0, sw = 0.0, ml = 0.0;
-  for (int k = 0; k < nz; ++k) {
-    const int ch = min(k / cpl, nchunk - 1);
-    if (k == ch * cpl) {
+  const long long og = (long long)i * ngrp * ny + j;
+  double *const t0 = tab + (long long)i * nchunk * TS * ny + j;
+  int ch = 0;
+  auto chunk_end = [&] {
+    double *t = t0 + (long long)ch * TS * ny;
+    t[0] = ml;
+    t[ny] = sw;
+    t[2 * ny] = w;
+  };
+  // a row k of the system that is neither the first nor the last
+  auto row = [&](double ak, double bk, double cc) {
+    const double z = zrcp<T>((bk + lam) - ak * dp);
+    dp = cc * z;
+    mp = (-ak * mp) * z;
+    if (PER) qp = (0.0 - ak * qp) * z;
+    sw = sw + w * mp;
+    w = -(dp * w);
+    ml = mp;
+  };
+  for (int g = 0; g < ngrp; ++g) {
+    const int k0 = g * gp;
+    if (ch + 1 < nchunk && k0 == (ch + 1) * cpl) {
+      chunk_end();
+      ++ch;
       mp = 1.0;
       w = 1.0;
       sw = 0.0;
       ml = 0.0;
     }
-    if (k % gp == 0) {
-      const long long o = ((long long)i * ngrp + k / gp) * ny + j;
-      ckd[o] = dp;
-      if (nchunk > 1) ckm[o] = mp;
-      if (per) ckq[o] = qp;
+    const long long o = og + (long long)g * ny;
+    ckd[o] = dp;
+    if (nchunk > 1) ckm[o] = mp;
+    if (PER) ckq[o] = qp;
+    if (k0 > 0 && k0 + gp < msys) {
+#pragma unroll 1
+      for (int l = 0; l < gp; l += H) {
+        double av[H], bv[H], cv[H];
+        slab_rows<H>(a + k0 + l, b + k0 + l, c + k0 + l, av, bv, cv);
+#pragma unroll
+        for (int r = 0; r < H; ++r) row(av[r], bv[r], cv[r]);
+      }
+      continue;
     }
-    if (k < msys) {
-      const double r2 = per ? ((k == msys - 1) ? -c[msys - 1] : ((k == 0) ? -a[0] : 0.0)) : 0.0;
+    for (int k = k0; k < min(k0 + gp, msys); ++k) {
+      if (k > 0 && k < msys - 1) {
+        row(a[k], b[k], c[k]);
+        continue;
+      }
+      const double r2 = PER ? (k == msys - 1 ? -c[msys - 1] : -a[0]) : 0.0;
       double dl = 0.0;
       if (k == 0) {
         const double z = zrcp<T>(b[0] + lam);
@@ -85,71 +126,87 @@ __global__ void __launch_bounds__(256)
         mp = 0.0;
         qp = r2 * z;
         dl = dp;
-      } else if (k < msys - 1) {
-        const double z = zrcp<T>((b[k] + lam) - a[k] * dp);
-        dp = c[k] * z;
-        mp = (-a[k] * mp) * z;
-        qp = (r2 - a[k] * qp) * z;
-        dl = dp;
       } else {
         const double z = (b[k] + lam) - a[k] * dp;
-        mp = (z != 0.0 && (per || !(pin && lam == 0.0))) ? (-a[k] * mp) / z : 0.0;
+        mp = (z != 0.0 && (PER || !(pin && lam == 0.0))) ? (-a[k] * mp) / z : 0.0;
         qp = (z != 0.0) ? (r2 - a[k] * qp) / z : 0.0;
       }
       sw = sw + w * mp;
       w = -(dl * w);
       ml = mp;
     }
-    const int ke = (ch == nchunk - 1) ? nz : (ch + 1) * cpl;
-    if (k == ke - 1) {
-      double *t = tab + ((long long)i * nchunk + ch) * TS * ny + j;
-      t[0] = ml;
-      t[ny] = sw;
-      t[2 * ny] = w;
-    }
   }
-  if (!per) return;
-  const int m = msys;  // nz - 1
-  double p2n = 0.0, p20 = 0.0, p2m1 = 0.0;
-  for (int g = ngrp - 1; g >= 0; --g) {
-    const int k0 = g * gp;
-    const long long o = ((long long)i * ngrp + g) * ny + j;
-    double dd[kZcMaxGroup], qq[kZcMaxGroup];
-    double d2 = ckd[o], q2 = ckq[o];
+  chunk_end();
+  if constexpr (PER) {
+    const int m = msys;  // nz - 1
+    double p2n = 0.0, p20 = 0.0, p2m1 = 0.0;
+    const long long last = og + (long long)(ngrp - 1) * ny;
+    double dn = ckd[last], qn = ckq[last];
+    for (int g = ngrp - 1; g >= 0; --g) {
+      const int k0 = g * gp;
+      double d2 = dn, q2 = qn;
+      // the next group's values, loaded ahead of this one's rows
+      const long long o = og + (long long)max(g - 1, 0) * ny;
+      dn = ckd[o];
+      qn = ckq[o];
+      constexpr int MG = GP ? GP : kZcMaxGroup;
+      double dd[MG], qq[MG];
+      if (GP && k0 > 0 && k0 + gp < m) {
 #pragma unroll
-    for (int l = 0; l < kZcMaxGroup; ++l) {
-      const int k = k0 + l;
-      if (l < gp && k < m) {
-        const double r2 = (k == m - 1) ? -c[m - 1] : ((k == 0) ? -a[0] : 0.0);
-        if (k == 0) {
-          const double z = zrcp<T>(b[0] + lam);
-          d2 = c[0] * z;
-          q2 = r2 * z;
-        } else if (k < m - 1) {
-          const double z = zrcp<T>((b[k] + lam) - a[k] * d2);
-          d2 = c[k] * z;
-          q2 = (r2 - a[k] * q2) * z;
-        } else {
-          const double z = (b[k] + lam) - a[k] * d2;
-          q2 = (z != 0.0) ? (r2 - a[k] * q2) / z : 0.0;
+        for (int h = 0; h < MG; h += H) {
+          double av[H], bv[H], cv[H];
+          slab_rows<H>(a + k0 + h, b + k0 + h, c + k0 + h, av, bv, cv);
+#pragma unroll
+          for (int l = 0; l < H; ++l) {
+            const double z = zrcp<T>((bv[l] + lam) - av[l] * d2);
+            d2 = cv[l] * z;
+            q2 = (0.0 - av[l] * q2) * z;
+            dd[h + l] = d2;
+            qq[h + l] = q2;
+          }
+        }
+#pragma unroll
+        for (int l = MG - 1; l >= 0; --l) p2n = qq[l] - dd[l] * p2n;
+      } else {
+#pragma unroll
+        for (int l = 0; l < MG; ++l) {
+          const int k = k0 + l;
+          if (l < gp && k < m) {
+            const double ak = a[k], bk = b[k], cc = c[k];
+            if (k == 0) {
+              const double z = zrcp<T>(bk + lam);
+              d2 = cc * z;
+              q2 = -ak * z;
+            } else if (k < m - 1) {
+              const double z = zrcp<T>((bk + lam) - ak * d2);
+              d2 = cc * z;
+              q2 = (0.0 - ak * q2) * z;
+            } else {
+              const double z = (bk + lam) - ak * d2;
+              q2 = (z != 0.0) ? (-cc - ak * q2) / z : 0.0;
+            }
+          }
+          dd[l] = d2;
+          qq[l] = q2;
+        }
+#pragma unroll
+        for (int l = MG - 1; l >= 0; --l) {
+          const int k = k0 + l;
+          if (l >= gp || k >= m) continue;
+          const double p2 = (k == m - 1) ? qq[l] : qq[l] - dd[l] * p2n;
+          p2n = p2;
+          if (k == m - 1) p2m1 = p2;
+          if (k == 0) p20 = p2;
         }
       }
-      dd[l] = d2;
-      qq[l] = q2;
+      // p2 of the plane after chunk ch - 1
+      if (ch > 0 && k0 == ch * cpl) {
+        t0[((long long)(ch - 1) * TS + 3) * ny] = p2n;
+        --ch;
+      }
     }
-#pragma unroll
-    for (int l = kZcMaxGroup - 1; l >= 0; --l) {
-      const int k = k0 + l;
-      if (l >= gp || k >= m) continue;
-      const double p2 = (k == m - 1) ? qq[l] : qq[l] - dd[l] * p2n;
-      p2n = p2;
-      if (k == m - 1) p2m1 = p2;
-      if (k == 0) p20 = p2;
-      if (k > 0 && k % cpl == 0 && k / cpl < nchunk)
-        tab[(((long long)i * nchunk + k / cpl - 1) * TS + 3) * ny + j] = p2;
-    }
+    den[(long long)i * ny + j] = ((b[m] + lam) + c[m] * p20) + a[m] * p2m1;
   }
-  den[(long long)i * ny + j] = ((b[m] + lam) + c[m] * p20) + a[m] * p2m1;
 }
 
 // Workgroups of the chunked P2 (*r2) and P3 (*r3) slab kernels that one CU
@@ -208,14 +265,20 @@ int build_zchunk_tables(double *mem, ZChunks *zc, int nx, int ny, int nz, int ms
   if (!per) ckq = den = nullptr;
   const int threads = 256;
   const long long blocks = ((long long)col + threads - 1) / threads;
-  if (elem_bytes == 8)
-    hipLaunchKernelGGL(k_zchunk_tables<double>, dim3((unsigned)blocks), dim3(threads), 0, s, ckd,
-                       ckm, ckq, tab, den, nx, ny, nz, msys, gp, cpl, nchunk, per ? 1 : 0, pin,
-                       lamx, lamy, a, b, c);
-  else
-    hipLaunchKernelGGL(k_zchunk_tables<float>, dim3((unsigned)blocks), dim3(threads), 0, s, ckd,
-                       ckm, ckq, tab, den, nx, ny, nz, msys, gp, cpl, nchunk, per ? 1 : 0, pin,
-                       lamx, lamy, a, b, c);
+  auto run = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(threads), 0, s, ckd, ckm, ckq, tab, den,
+                       nx, ny, nz, msys, gp, cpl, nchunk, pin, lamx, lamy, a, b, c);
+  };
+  auto by_group = [&](auto t, auto p) {
+    using T = decltype(t);
+    constexpr bool P = decltype(p)::value;
+    if (gp == 16) run(&k_zchunk_tables<T, P, 16>);
+    else if (gp == 8) run(&k_zchunk_tables<T, P, 8>);
+    else if (gp == 4) run(&k_zchunk_tables<T, P, 4>);
+    else run(&k_zchunk_tables<T, P, 0>);
+  };
+  if (elem_bytes == 8) per ? by_group(double(), std::true_type()) : by_group(double(), std::false_type());
+  else per ? by_group(float(), std::true_type()) : by_group(float(), std::false_type());
   FL_HIP(hipGetLastError());
   *zc = ZChunks{nchunk, cpl, ngrp, ckd, ckm, ckq, tab, den, side};
   return FLUTAS_OK;
