@@ -140,6 +140,11 @@ struct ChunkSet {
   int n = 1;
   ZChunks zc{};
   double *mem = nullptr;
+  bool own = true;  // mem is an allocation of its own
+  void free() {
+    if (mem && own) (void)hipFree(mem);
+    *this = ChunkSet{};
+  }
 };
 
 struct flutas_psolve {
@@ -224,12 +229,12 @@ void release(flutas_psolve *h) {
                    (void **)&h->d_b, (void **)&h->d_c, (void **)&h->d_rhsbx,
                    (void **)&h->d_rhsby, (void **)&h->d_rhsbz, (void **)&h->W64,
                    (void **)&h->W32, (void **)&h->TK, (void **)&h->F,
-                   (void **)&h->R32, (void **)&h->part, (void **)&h->CK, (void **)&h->zcs.mem,
-                   (void **)&h->zcs32.mem}) {
+                   (void **)&h->R32, (void **)&h->part, (void **)&h->CK}) {
     if (*p) (void)hipFree(*p);
     *p = nullptr;
   }
-  h->zcs = h->zcs32 = ChunkSet{};
+  h->zcs.free();
+  h->zcs32.free();
   for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
   h->ev.clear();
   if (h->nf_host) (void)hipHostFree(h->nf_host);
@@ -370,32 +375,46 @@ void chunk_shape(int nz, int gp, int n, int *cpl, int *nch) {
 // Chunks per x-slab for the z-chunked slab passes of a chain of elem-byte
 // values: n = 1 turns them off.  The planes are cut at multiples of the plane
 // group into n chunks (fewer when nz is short; the last chunk runs to nz and
-// holds two planes or more), and the tables are computed for that chain.
-int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
-  z = ChunkSet{};
-  if (!h->fused || (n == 1 && !h->gy)) return FLUTAS_OK;
-  const int gp = h->gy ? general_group_planes(h->ny) : fused_group_planes(h->ny, elem);
-  const int nz = h->nz;
+// holds two planes or more).  doubles: values of the tables, 0 for whole slabs.
+struct ChunkShape {
+  int gp = 0, cpl = 0, n = 1;
+  size_t doubles = 0;
+};
+ChunkShape chunk_tables(const flutas_psolve *h, int elem, int n) {
+  ChunkShape c;
+  if (!h->fused || (n == 1 && !h->gy)) return c;
+  c.gp = h->gy ? general_group_planes(h->ny) : fused_group_planes(h->ny, elem);
+  chunk_shape(h->nz, c.gp, n, &c.cpl, &c.n);
+  if (c.n < 2 && !h->gy) return ChunkShape{};
+  c.doubles = zchunk_doubles(h->nx, h->ny, (h->nz + c.gp - 1) / c.gp, c.n, h->cbc[4] == 'P');
+  return c;
+}
+// Computes a chain's tables in mem, on stream s.
+int fill_chunks(flutas_psolve *h, ChunkSet &z, int elem, const ChunkShape &c, double *mem,
+                hipStream_t s) {
   const int per = (h->cbc[4] == 'P');
   const int pin = (h->cbc[4] == 'N' && h->cbc[5] == 'N') || per;
-  int cpl, nch;
-  chunk_shape(nz, gp, n, &cpl, &nch);
-  if (nch < 2 && !h->gy) return FLUTAS_OK;
-  const int ngrp = (nz + gp - 1) / gp;
-  const size_t nd = zchunk_doubles(h->nx, h->ny, ngrp, nch, per != 0);
-  FL_HIP(hipMalloc((void **)&z.mem, nd * sizeof(double)));
-  int rc = build_zchunk_tables(z.mem, &z.zc, h->nx, h->ny, nz, per ? nz - 1 : h->nzs, gp, cpl, nch,
-                               per != 0, pin, elem, h->d_lamx, h->d_lamy, h->d_a, h->d_b, h->d_c,
-                               nullptr);
+  FL_TRY(build_zchunk_tables(mem, &z.zc, h->nx, h->ny, h->nz, per ? h->nz - 1 : h->nzs, c.gp, c.cpl,
+                             c.n, per != 0, pin, elem, h->d_lamx, h->d_lamy, h->d_a, h->d_b,
+                             h->d_c, s));
+  z.mem = mem;
+  z.n = c.n;
+  return FLUTAS_OK;
+}
+int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
+  z = ChunkSet{};
+  const ChunkShape c = chunk_tables(h, elem, n);
+  if (!c.doubles) return FLUTAS_OK;
+  double *mem = nullptr;
+  FL_HIP(hipMalloc((void **)&mem, c.doubles * sizeof(double)));
+  int rc = fill_chunks(h, z, elem, c, mem, nullptr);
   if (rc == FLUTAS_OK && hipDeviceSynchronize() != hipSuccess)
     rc = fail(FLUTAS_EDEVICE, "z chunk tables");
   if (rc) {
-    (void)hipFree(z.mem);
+    (void)hipFree(mem);
     z = ChunkSet{};
-    return rc;
   }
-  z.n = nch;
-  return FLUTAS_OK;
+  return rc;
 }
 
 // Default chunking: the count that fills the GPU's workgroup slots best
@@ -464,16 +483,14 @@ int default_zchunks(const flutas_psolve *h, int elem) {
   return best;
 }
 
-// The tables of solve_f32 on an FP64 plan: its slab passes fill the GPU no
+// The chunk count of solve_f32 on an FP64 plan: its slab passes fill the GPU no
 // better than the FP64 ones (solve_f32 on whole slabs and in the default chunks:
 // 128^3 109 and 58 us, 256^3 269 and 175, 256x256x512 periodic 578 and 346,
 // 48x64x364 195 and 51; 512^3 stays at one chunk).  Whole slabs serve it
-// where the memory for them is short.
+// where the memory for the tables is short.
+int chunks32(const flutas_psolve *h) { return h->zreq ? h->zreq : default_zchunks(h, 4); }
 void build_chunks32(flutas_psolve *h) {
-  if (build_chunks(h, h->zcs32, 4, h->zreq ? h->zreq : default_zchunks(h, 4)) != FLUTAS_OK) {
-    (void)hipGetLastError();
-    h->zcs32 = ChunkSet{};
-  }
+  if (build_chunks(h, h->zcs32, 4, chunks32(h)) != FLUTAS_OK) (void)hipGetLastError();
 }
 
 int plan_elem(const flutas_psolve *h) { return h->precision == FLUTAS_FP64 ? 8 : 4; }
@@ -487,9 +504,8 @@ int set_zchunks(flutas_psolve *h, int n) {
   const int before = h->zcs.n;
   if (h->zcs.mem || h->zcs32.mem) {
     FL_HIP(hipDeviceSynchronize());
-    (void)hipFree(h->zcs.mem);
-    (void)hipFree(h->zcs32.mem);
-    h->zcs = h->zcs32 = ChunkSet{};
+    h->zcs.free();
+    h->zcs32.free();
   }
   const int rc = build_chunks(h, h->zcs, plan_elem(h), n);
   if (rc) {
@@ -578,6 +594,30 @@ int solve_fp64(flutas_psolve *h, const double *f, double *p, hipStream_t s) {
   return FLUTAS_OK;
 }
 
+// The FP32 work field of an FP64 plan and, behind it in one allocation, the chunk
+// tables of its chain, computed on the solve's own stream ahead of it.  First FP32
+// solve of a new plan, in whole slabs, with an allocation for the tables and a wait
+// for the device, and so: 256^3 346, 343, 265 us, 128^3 140, 142, 97, 200x100x300
+// periodic z 310, 410, 248.
+int make_work32(flutas_psolve *h, hipStream_t s) {
+  const bool tables = h->fused && !h->gy;
+  const ChunkShape c = tables ? chunk_tables(h, 4, chunks32(h)) : ChunkShape{};
+  h->has32 = tables;
+  if (c.doubles) {
+    const int q = line_pitch(h->ny, 4);
+    const size_t field = ((size_t)h->nx * q * h->nz * sizeof(float) + 255) & ~size_t(255);
+    if (hipMalloc((void **)&h->W32, field + c.doubles * sizeof(double)) == hipSuccess) {
+      h->pitch32 = q;
+      h->zcs32.own = false;
+      return fill_chunks(h, h->zcs32, 4, c,
+                         reinterpret_cast<double *>(reinterpret_cast<char *>(h->W32) + field), s);
+    }
+    (void)hipGetLastError();
+  }
+  FL_HIP(alloc_work(h, &h->W32, &h->pitch32, !h->fused));
+  return FLUTAS_OK;
+}
+
 // The solve of an FP32 field (a FluTAS build with _SINGLE_PRECISION, rp =
 // FP32: src/types.f90:6-12), in place or out of place: the FP32 chain of
 // the refined mode (FP32 transforms, FP64 z elimination) once, no
@@ -585,11 +625,7 @@ int solve_fp64(flutas_psolve *h, const double *f, double *p, hipStream_t s) {
 // solve in FP32.  The FP32 work field and the chunk tables are made on
 // first use when the plan is an FP64 one.
 int solve_f32(flutas_psolve *h, const float *f, float *p, hipStream_t s) {
-  if (!h->W32) FL_HIP(alloc_work(h, &h->W32, &h->pitch32, !h->fused));
-  if (!h->has32 && h->fused && !h->gy && h->precision == FLUTAS_FP64) {
-    h->has32 = true;
-    build_chunks32(h);
-  }
+  if (!h->W32) FL_TRY(make_work32(h, s));
   const Geo q = halo_geo(h);
   ++h->seq;
   FL_TRY((spectral<float, float, float>(h, f + q.interior, true, p + q.interior, 0, h->W32, s,

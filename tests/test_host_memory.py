@@ -195,3 +195,32 @@ if not {kw}:
     assert solve32(p, d32) == 0 and sim.sim_count(2) == 0
     p.destroy()
 """, tmp_path)
+
+
+@pytest.mark.parametrize("ng,cbc", [((64, 64, 96), "PPDDNN"), ((90, 128, 200), "PPDDPP"),
+                                    ((64, 154, 96), "PPDDNN"), ((512, 512, 8), "PPPPNN")])
+def test_first_f32_solve_stays_on_its_stream(tmp_path, ng, cbc):
+    """One allocation, no wait for the device (other streams go on), every
+    launch on the solve's stream; the second solve is the four passes."""
+    hipsim.run(f"""
+ng = {ng}
+p, d = plan(ng, "{cbc}"), field(ng, np.float32)
+api.lib.flutas_set_stream(C.c_void_p(0x1234))
+sim.sim_reset()
+assert solve32(p, d) == 0
+assert sim.sim_count(0) == 1 and sim.sim_count(1) == 0, (sim.sim_count(0), sim.sim_count(1))
+first = launches()
+assert all(l[4] == 0x1234 for l in first)
+assert len(first) == 4 + any("k_zchunk_tables" in l[0] for l in first)
+sim.sim_reset()
+assert solve32(p, d) == 0
+assert launches() == first[-4:]
+assert sim.sim_count(0) == sim.sim_count(1) == 0
+# another count, then the plan's own again
+for n in (3, 0):
+    p.set_zchunks(n)
+    assert solve32(p, d) == 0 and sim.sim_count(2) == 0
+p.destroy()
+d.free()
+assert sim.sim_used() == 0
+""", tmp_path)
