@@ -249,6 +249,7 @@ static bool has_prime(const RadixList &rl) {
     if (rl.r[q] > 13) return true;
   return false;
 }
+bool general_has_prime(int n) { return general_supported(n) && has_prime(y_shape(n).rl); }
 
 // Dynamic LDS beyond 64 KiB has to be asked for.  The limit belongs to the
 // kernel, which all plans and threads of the process share: every launch asks

@@ -264,6 +264,7 @@ int launch_zy_bwd(const LineTables &ty, int kind, T *Wt, WStride ws,
 // plan.  The passes take the arguments of the compiled ones; the slab passes
 // are always z-chunked (zc.nchunk >= 1), in groups of general_group_planes(ny).
 bool general_supported(int n);
+bool general_has_prime(int n);  // its radix list holds a prime above 13
 int general_group_planes(int ny);
 int general_slab_residency(int ny, int elem_bytes, int periodic, int *r2, int *r3);
 int build_general_tables(LineTables &tab, int n);

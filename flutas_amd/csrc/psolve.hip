@@ -748,6 +748,16 @@ int setup_device(flutas_psolve *h, bool lean) {
   const char *env = std::getenv("FLUTAS_UNFUSED");
   const bool tile_kinds = fused_forward_kind(h->kinds[0]) && fused_forward_kind(h->kinds[2]);
   const bool gx = !fused_supported(h->nx), gy = !fused_supported(h->ny);
+  // Both lengths general, few values and at most 8 planes: the five short launches
+  // of the line path are done before the general passes have staged their tables
+  // (FP64, FP32 solves of 2x2x4 periodic z 31, 27 against 35, 31 us, 60x2x4 37, 33
+  // against 44, 40, 360x2x4 43, 39 against 49, 42; from 16 planes on the elimination
+  // turns it, 6x6x16 41, 39 against 38, 36, and 90x90x4 takes 61 against 50).  A prime
+  // above 13 the line path sums 20 times slower, and the refined mode's checks cost
+  // it more than the passes save.
+  if (fp64 && gx && gy && h->nz <= 8 && N <= 8192 && !general_has_prime(h->nx) &&
+      !general_has_prime(h->ny))
+    lean = true;
   h->fused = (!gx || (general_supported(h->nx) && !lean)) &&
              (!gy || (general_supported(h->ny) && !lean)) && h->nz >= 3 && tile_kinds &&
              !(env && env[0] == '1');

@@ -6,7 +6,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from cases import z_metrics
+from cases import interior, relmax, z_metrics
 
 pytestmark = pytest.mark.gpu
 
@@ -50,4 +50,27 @@ def test_refined_nonfinite_gives_the_right_hand_side_back(api, oracle, ng, bad):
             call()
         assert e.value.code == api.FLUTAS_ENONFINITE
         np.testing.assert_array_equal(d.to_host(), f)
+    plan.destroy()
+
+
+@pytest.mark.parametrize("ng", [(2, 2, 4), (6, 10, 4), (90, 2, 8), (2, 90, 6), (30, 30, 8), (360, 2, 4),
+                                (2, 1000, 4), (30, 34, 8), (90, 30, 4), (60, 60, 10)])
+@pytest.mark.parametrize("cbc", ["PPDDNN", "NDPPPP"])
+def test_few_planes_match_oracle(api, oracle, ng, cbc):
+    """Both sides of the rule for few values in few planes, FP64 and FP32
+    fields, to the bounds of every length."""
+    dzc, dzf, dzci, dzfi, _, _ = z_metrics(oracle, ng[2], 0.0, 1.1)
+    dli = (ng[0] / 1.0, ng[1] / 0.8, ng[2] / 1.1)
+    f = np.zeros(tuple(n + 2 for n in ng), order="F")
+    f[1:-1, 1:-1, 1:-1] = np.random.default_rng(sum(ng)).standard_normal(ng).astype(np.float32)
+    ref = f.copy(order="F")
+    oracle.Solver(ng, dli, dzci, dzfi, cbc).solve(ref, pin_gauge=True)
+    plan = api.PoissonPlan(ng, dli, dzci, dzfi, cbc)
+    d, p = api.DeviceArray.from_host(f), api.DeviceArray(f.shape)
+    p.zero()
+    plan.solve_into(d, p)
+    assert relmax(interior(p.to_host()), interior(ref)) <= 1e-12
+    s = api.DeviceArray.from_host(np.asfortranarray(f.astype(np.float32)))
+    assert _solve32(api, plan, s) == 0
+    assert relmax(interior(s.to_host().astype(np.float64)), interior(ref)) <= 1e-4
     plan.destroy()

@@ -224,3 +224,20 @@ p.destroy()
 d.free()
 assert sim.sim_used() == 0
 """, tmp_path)
+
+
+@pytest.mark.parametrize("ng,kw,line", [
+    ((2, 2, 4), "{}", True), ((60, 6, 8), "{}", True), ((30, 34, 8), "{}", False),
+    ((60, 6, 10), "{}", False), ((90, 90, 4), "{}", False), ((64, 6, 4), "{}", False),
+    ((6, 64, 4), "{}", False), ((60, 6, 8), "dict(precision=32)", False)])
+def test_route_of_small_plans(tmp_path, ng, kw, line):
+    """Few values in at most 8 planes, both lengths without a compiled plan and
+    without a large prime: the line path; else the four passes."""
+    hipsim.run(f"""
+ng = {ng}
+p, f, g = plan(ng, **{kw}), field(ng), field(ng)
+sim.sim_reset()
+api.lib.flutas_psolve_solve_into(C.c_void_p(p._h), f.c, g.c)
+names = [l[0] for l in launches()]
+assert any("k_lines" in n for n in names) == {line}, names
+""", tmp_path)
