@@ -74,3 +74,63 @@ def test_few_planes_match_oracle(api, oracle, ng, cbc):
     assert _solve32(api, plan, s) == 0
     assert relmax(interior(s.to_host().astype(np.float64)), interior(ref)) <= 1e-4
     plan.destroy()
+
+
+def _random_case(oracle, ng, cbc, seed):
+    dzc, dzf, dzci, dzfi, _, _ = z_metrics(oracle, ng[2], 0.0, 1.1)
+    dli = (ng[0] / 1.0, ng[1] / 0.8, ng[2] / 1.1)
+    f = np.zeros(tuple(n + 2 for n in ng), order="F")
+    f[1:-1, 1:-1, 1:-1] = np.random.default_rng(seed).standard_normal(ng).astype(np.float32)
+    ref = f.copy(order="F")
+    oracle.Solver(ng, dli, dzci, dzfi, cbc).solve(ref, pin_gauge=True)
+    return f, interior(ref), dzci, dzfi, dli
+
+
+@pytest.mark.parametrize("ng", [(90, 512, 18), (36, 512, 20), (254, 512, 6), (6, 512, 40)])
+@pytest.mark.parametrize("cbc", ["NNDDNN", "PPNDPP"])
+def test_general_x_with_a_blocked_work_field(api, oracle, ng, cbc):
+    """512-point y lines keep the FP64 work field in blocks of up to 8 slabs (2
+    for 90 and 254, 4 for 36): the general x passes write and read it."""
+    f, ref, dzci, dzfi, dli = _random_case(oracle, ng, cbc, 5)
+    plan = api.PoissonPlan(ng, dli, dzci, dzfi, cbc)
+    d, p = api.DeviceArray.from_host(f), api.DeviceArray(f.shape)
+    for n in (0, 1, 2):
+        plan.set_zchunks(n)
+        p.zero()
+        plan.solve_into(d, p)
+        assert relmax(interior(p.to_host()), ref) <= 1e-12
+    plan.destroy()
+
+
+@pytest.mark.parametrize("n", [22, 34, 254, 514, 1020, 1026, 2046])
+@pytest.mark.parametrize("axis", [0, 1])
+def test_f32_and_refined_long_and_prime_lengths(api, oracle, n, axis):
+    """The FP32 chain at lists with a prime, tiles of fewer lines and slab groups
+    of two and four columns a thread: FP32 fields to 1e-4, refined solves to
+    their residual and 1e-9, as at every length.  20 lines: one full tile of 16
+    and a partial one."""
+    ng = (n, 20, 38) if axis == 0 else (6, n, 38)
+    cbc = "NDPPNN" if axis == 0 else "PPDDPP"
+    f, ref, dzci, dzfi, dli = _random_case(oracle, ng, cbc, n)
+    plan = api.PoissonPlan(ng, dli, dzci, dzfi, cbc)
+    s = api.DeviceArray.from_host(np.asfortranarray(f.astype(np.float32)))
+    assert _solve32(api, plan, s) == 0
+    assert relmax(interior(s.to_host().astype(np.float64)), ref) <= 1e-4
+    plan.destroy()
+    plan = api.PoissonPlan(ng, dli, dzci, dzfi, cbc, precision=api.FP32_REFINE, tol=1e-9)
+    d, p = api.DeviceArray.from_host(f), api.DeviceArray(f.shape)
+    p.zero()
+    plan.solve_into(d, p)
+    assert plan.stats()[1] <= 1e-9
+    assert relmax(interior(p.to_host()), ref) <= 1e-9
+    plan.destroy()
+
+
+@pytest.mark.parametrize("ng", [(36, 60, 70), (22, 300, 40), (90, 520, 22)])
+def test_chunk_counts_stay_within_what_is_asked(api, oracle, ng):
+    _, _, dzci, dzfi, _, _ = z_metrics(oracle, ng[2], 0.0, 1.0)
+    plan = api.PoissonPlan(ng, tuple(float(n) for n in ng), dzci, dzfi, "PPDDNN")
+    assert 1 <= plan.set_zchunks(0) <= 8
+    for n in range(1, 9):
+        assert 1 <= plan.set_zchunks(n) <= n
+    plan.destroy()
