@@ -981,24 +981,38 @@ constexpr int slab_threads() {
 // round (tile::lane_id): true where the registers they would hold keep a
 // workgroup from the CU that the LDS has room for, or push values into the
 // accumulation registers; false where the LDS or 512 threads set the residency
-// and the instructions only cost time.  Measured, addresses kept / computed
-// anew (us):
-//   FP64 P2, P3   200^3 periodic 61, 129 / 58, 70 (kept: one workgroup a CU);
-//                 192^3 62, 76 / 50, 54; 384x384x200 periodic P3 366 / 212;
-//                 400x800x200 509, 654 / 368, 402;
-//                 512^3 434, 453 / 491, 495; 400^3 P2 310 / 340
-//   FP32 P3       384^3 481 / 255, 768x768x256 1081 / 636 (its P2 keeps up only
-//                 so: 649 / 484), 400^3 570 / 361;
-//                 512^3 327 / 367; 1024x1024x128 periodic 805 / 532
+// and the instructions only cost time.  Which it is turns on a few registers of
+// each kernel, so every one was timed both ways (x of 64, 256 and 1024 slabs, both
+// z closures, 1, 4 and the default number of chunks), and a kernel computes its
+// addresses anew where that was ever more than 1% faster.  Measured, addresses
+// kept / computed anew (us):
+//   FP64 P2, P3   256^3 in 4 chunks 77, 90 / 82, 93; 1024x256x256 244, 284 / 274, 308;
+//                 1024x192x256 216, 229 / 240, 252; 200^3 periodic z in 4 chunks 65,
+//                 119 / 72, 81; 1024x80x256 in 4 chunks 150, 191 / 127, 155;
+//                 400^3 P3 346 / 368, 640x640x128 P3 310 / 330;
+//                 512x800x128 in 4 chunks 397, 468 / 306, 327;
+//                 512x512x256 219, 300 / 244, 300
+//   FP32 P2, P3   256^3 in 4 chunks 56, 73 / 51, 55; 400x400x200 P3 244 / 160;
+//                 512x768x128 P2, P3 139, 292 / 165, 191; 512x2048x64 P3 361 / 382
 // A batch has workgroups of all lengths to fill a CU with and keeps its
 // addresses (64 problems 4547 / 4662).
 template <typename T, int NC, bool PER, bool BWD, bool CHUNK>
 constexpr bool slab_opaque() {
-  constexpr bool f32 = sizeof(T) == 4;
-  if (NC <= 160 || NC == 400 || ((NC == 512 || NC == 256) && f32 && PER)) return true;
-  if (!BWD) return f32 && (NC == 192 || NC == 384 || (NC == 200 && CHUNK) || (NC == 320 && PER));
-  if (NC == 384) return f32 || PER;
-  return NC == 192 || NC == 200 || NC == 320 || (NC == 1024 && f32);
+  // bits 0 to 3: P2 of whole slabs, with periodic z, of chunks, with periodic z;
+  // bits 4 to 7: P3
+  struct Row {
+    int n;
+    unsigned f64, f32;
+  };
+  constexpr Row rows[] = {
+      {32, 0x88, 0xcc},  {48, 0x5f, 0xcc},  {64, 0xff, 0xcc},  {80, 0x5f, 0xfc},  {96, 0x4c, 0xdf},
+      {100, 0xdf, 0x5f}, {128, 0x6c, 0xdf}, {160, 0x60, 0xdf}, {192, 0x00, 0xdf}, {200, 0x80, 0xdf},
+      {256, 0x00, 0xff}, {320, 0xcc, 0xfe}, {384, 0x80, 0xff}, {400, 0x00, 0xfc}, {512, 0x00, 0xa2},
+      {640, 0x00, 0xea}, {768, 0x80, 0xfe}, {800, 0xff, 0xff}, {1024, 0x00, 0xaa}, {2048, 0x00, 0x00}};
+  for (const Row &r : rows)
+    if (r.n == 2 * NC)
+      return ((sizeof(T) == 4 ? r.f32 : r.f64) >> (4 * BWD + 2 * CHUNK + PER)) & 1;
+  return false;
 }
 
 // Threads of a batched slab workgroup (lines of up to 256 points): one

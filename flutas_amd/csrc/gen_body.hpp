@@ -200,8 +200,6 @@ template <typename T, int S, int R>
 __device__ __forceinline__ void dftr(cx<T> *v) {
   if constexpr (R == 6) dgood<T, S, 2, 3>(v);
   else if constexpr (R == 10) dgood<T, S, 2, 5>(v);
-  else if constexpr (R == 12) dgood<T, S, 4, 3>(v);
-  else if constexpr (R == 15) dgood<T, S, 3, 5>(v);
   else if constexpr (R == 9) d9<T, S>(v);
   else if constexpr (R == 7 || R == 11 || R == 13) dprime<T, S, R>(v);
   else tile::dft<T, S, R>(v);

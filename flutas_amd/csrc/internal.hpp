@@ -381,7 +381,8 @@ int launch_flag_nonfinite(const double *f_halo, int nx, int ny, int nz, int *fla
                           hipStream_t s);
 // partial count of launch_residual and launch_absmax
 size_t residual_blocks(int nx, int ny, int nz);
-// out[0] = max of n partial maxima (single workgroup)
+// out[0] = max of the n0 partial maxima part0 and, where n1 > 0, out[1] = that of
+// the n1 of part1 (a workgroup each)
 int launch_reduce_max(const double *part0, int n0, const double *part1, int n1, double *out,
                       hipStream_t s);
 
