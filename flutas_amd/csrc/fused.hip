@@ -121,12 +121,19 @@ int launch_x_fwd(const LineTables &tx, int kind, const Tin *in, long long is1,
 }
 
 // FP64 outputs above this many bytes, in lines of 512 and 1024 points, are stored
-// from aligned lanes (x_bwd_tile): HBM takes whole memory lines sooner (P4 of 512^3
-// 462 -> 429 us, 1024x1024x512 2349 -> 2262), the cache does not mind and the
-// further lanes cost time (1024x256x128 137 -> 142 us, 512x512x160 143 -> 142; lines
-// of 640, 768 and 800 points 380 -> 406, 518 -> 554, 270 -> 289; FP32 transforms
-// 362 -> 376).
-constexpr double kAlignBytes = 512e6;
+// from aligned lanes (x_bwd_tile): HBM takes whole memory lines sooner, the cache
+// does not mind and the further lanes cost time.  P4, lanes from the line's start /
+// aligned (us): 512-point lines 512x400x320 209 / 184, 512x512x256 228 / 213,
+// 512x768x320 430 / 388, 512^3 452 / 416, 512x512x1000 889 / 821 (336 MB 141 / 134, but
+// the same grid 143 / 142 in another run); 1024-point lines, whose tile is 8 of them
+// and not 16, gain only from 2 GB on: 1024x512x256 546 / 551, 1024x768x200 645 / 658,
+// 1024x1024x256 (2.1 GB) 1095 / 1087, 1024x1024x512 2349 / 2262.  Lines of 640, 768 and
+// 800 points were slower aligned (380 / 406, 518 / 554, 270 / 289; 8 lines a tile too), as
+// were FP32 transforms (362 / 376).
+template <int NC>
+constexpr double align_bytes() {
+  return NC == 256 ? 512e6 : 2e9;
+}
 template <typename T, typename Tout>
 int launch_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws,
                  Tout *out, long long os1, long long os2, int ny, int nz,
@@ -143,7 +150,7 @@ int launch_x_bwd(const LineTables &tx, int kind, const T *Wt, WStride ws,
                          pl.tw, th, tq);
     };
     if constexpr ((NC == 256 || NC == 512) && sizeof(T) == 8) {
-      if (!accumulate && (double)tx.n * ny * nz * sizeof(Tout) > kAlignBytes) {
+      if (!accumulate && (double)tx.n * ny * nz * sizeof(Tout) > align_bytes<NC>()) {
         run(&k_x_bwd<T, Tout, NC, TJ, NT, false, true>);
         FL_HIP(hipGetLastError());
         return FLUTAS_OK;

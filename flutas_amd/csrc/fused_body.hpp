@@ -274,7 +274,7 @@ __device__ __forceinline__ void x_fwd_tile(const Tin *__restrict__ in, long long
 // Inverse of P1: out(i, j, k) = scale * r2r^-1 (x) (+ out when ACC).
 // ALIGN: lanes start at the 128-byte boundary before a line of out, which the
 // halo puts anywhere, so that each wave stores whole memory lines; a line then
-// takes n and 128 bytes of lanes (kAlignBytes says where that pays).
+// takes n and 128 bytes of lanes (align_bytes says where that pays).
 template <typename T, typename Tout, int NC, int TJ, int NT, bool ACC, bool ALIGN = false>
 __device__ __forceinline__ void x_bwd_tile(const T *__restrict__ Wt, WStride ws,
                                            Tout *__restrict__ out,
