@@ -986,10 +986,12 @@ static int check_dims(int nx, int ny, int nz) {
 // Bound by the x faces: their points lie in a line's end and the next one's
 // start, one or two 128-byte lines of memory per grid line and field, so a
 // thread takes all points of a line; the y and z faces are rows along x.
-// In a step of 128^3 the two velocity calls take 9 us each, 17 with every point
-// walking the stages; boundp of 256x256x512 periodic takes 10 us a call, 25 in
-// six face launches; the whole step 191 -> 171 us (128^3, a recorded graph) and
-// 2123 -> 2024 us (256x256x512 call by call).
+// In a step of 128^3 the two velocity calls take 8.6 us each, 17 with every point
+// walking the stages.  256x256x512 periodic, called back to back: boundp 10 us a
+// call, 24 in six face launches, bounduvw 35, 41 with the walk; in a step, whose
+// other calls have put the faces out of the caches, 15 to 18 and 42 to 48.  The
+// whole step 191 -> 171 us (128^3, a recorded graph) and 2123 -> 2024 us
+// (256x256x512 call by call).
 template <typename T>
 struct HaloRule {
   T A;

@@ -14,7 +14,7 @@
 //
 // Against the compiled lengths (measured with compiled lengths forced onto
 // these kernels) an element costs about 1.5 times the instructions: 512^3 P1
-// 389 -> 695, P2 440 -> 615 us, 256^3 53 -> 71, 83 -> 86 us, so the compiled
+// 389 -> 695, P2 440 -> 615 us, 256^3 53 -> 71, 77 -> 86 us, so the compiled
 // plans stay.  Against the five-pass line path, which ran these lengths
 // before: 360x300x240 1.68 -> 0.61 ms (2.7 TB/s; P1 125, P2 181, P3 185,
 // P4 137 us), 210x154x90 0.36 -> 0.10 ms, 450x450x300 4.0 -> 1.2 ms.

@@ -433,19 +433,18 @@ int build_chunks(flutas_psolve *h, ChunkSet &z, int elem, int n) {
 // FP32 chain of the refined mode pays 5% of score per chunk beyond the
 // first: its chunk tables and side arrays stay FP64 against half the field
 // bytes, so a chunk costs it relatively more (refined 256x256x512
-// periodic: 1/2/3/4/6/8 chunks 1.71, 1.30, 1.36, 1.31, 1.37, 1.34 ms; the
-// unpenalised score took 6, the penalised one takes 2; refined 128^3:
-// 0.309, 0.244, 0.230, 0.207, 0.249, 0.225 ms, 4 either way).
+// periodic: 1/2/3/4/6/8 chunks 1.54, 1.21, 1.14, 1.15, 1.18, 1.17 ms, 3 taken;
+// refined 128^3 1/2/3/4/7/8: 0.240, 0.179, 0.171, 0.155, 0.162, 0.147 ms, 4 taken).
 // Measured FP64 solves (ms for 1/2/3/4/6/8 chunks; * the count taken):
-//   768x768x256 NN-z      2.71  2.65* 2.68  2.67  2.75  2.76
-//   640x640x320 NN-z      2.65  2.46  2.48  2.42* 2.51  2.50
-//   640x640x256 periodic  2.24  2.02  2.06  2.01* 2.07  2.10
-//   384x768x256 DD-z      1.41  1.36  1.39  1.28* 1.34  1.33
-//   512^3 NN-z            1.69* 1.71  1.71  1.81  1.75  1.77
-//   1024x1024x512 NN-z    8.77* 9.47  9.46  9.56  9.68  9.76
-//   256x256x512 periodic  0.70  0.53* 0.56  0.59  0.57  0.57
-//   400^3 NN-z            1.09  1.18  1.10  1.13  1.13  1.16  (5 taken: 1.06)
-// and at 128^3: 0.114, 0.082 (2), 0.069 (4, taken), 0.078 (8).
+//   768x768x256 NN-z      2.72  2.66* 2.70  2.68  2.76  2.77
+//   640x640x320 NN-z      2.58  2.42  2.44  2.38* 2.47  2.47
+//   640x640x256 periodic  2.19  1.99  2.02  1.97* 2.04  2.07
+//   384x768x256 DD-z      1.42  1.36  1.39  1.29* 1.34  1.34
+//   512^3 NN-z            1.76* 1.77  1.77  1.90  1.80  1.83
+//   1024x1024x512 NN-z    8.92* 9.64  9.61  9.74  9.84  9.95
+//   256x256x512 periodic  0.65  0.49* 0.55  0.56  0.54  0.54
+//   400^3 NN-z            1.04  1.14  1.07  1.11  1.10  1.13  (5 taken: 1.04)
+// and at 128^3: 0.095, 0.071 (2), 0.058 (4, taken), 0.067 (8).
 int default_zchunks(const flutas_psolve *h, int elem) {
   if (!h->fused) return 1;
   const int per = (h->cbc[4] == 'P');

@@ -153,8 +153,10 @@ int flutas_psolve_time_stage(flutas_psolve *h, const double *f, double *p, int s
  * (the count that best fills the GPU's workgroup slots over the two slab
  * passes, from the CU count and the kernels' occupancy, with chunks of 32
  * planes or more unless the workgroups do not reach the CUs); n = 1 walks
- * whole slabs.  FP32 solves on an FP64 plan follow n, or their own default.  The count may come out lower than n for
- * a short z.  Results equal the whole-slab walk's to rounding; the pivots
+ * whole slabs.  FP32 solves on an FP64 plan follow n, or their own default.
+ * The count may come out lower than n for a short z, and is 1 on the line
+ * path; where the tables of n do not fit the device the call fails and the
+ * plan keeps the count it had.  Results equal the whole-slab walk's to rounding; the pivots
  * stay the reference's bit for bit.  Changing the count frees the tables a
  * recorded graph of this plan's solve refers to: record again after it.
  * flutas_psolve_zchunks reads the count in use. */
